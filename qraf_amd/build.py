@@ -30,6 +30,11 @@ FLAGS = ["-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", f"--offload-arch={AR
          "-Xclang", "-packed-fp32-ops", "-Wno-unused-command-line-argument", "-I", os.path.join(ROOT, "include")]
 
 
+# The 32x32 GEMM keeps its accumulators in VGPRs (its scale FMAs read and
+# write them); the compiler's default at one wave per SIMD puts MFMA results
+# in AGPRs, a copy per register around every FMA.
+FILE_FLAGS = {"qgemm_wide.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+
 CXX = os.environ.get("CXX", "g++")
 CXXFLAGS = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-I", os.path.join(ROOT, "include")]
 
@@ -39,7 +44,7 @@ def _compile(src: str) -> str:
     if src.endswith(".cpp"):  # host-only sources (no HIP): the plain C++ compiler
         cmd = [CXX, *CXXFLAGS, "-c", src, "-o", obj]
     else:
-        cmd = [HIPCC, *FLAGS, "-c", src, "-o", obj]
+        cmd = [HIPCC, *FLAGS, *FILE_FLAGS.get(os.path.basename(src), []), "-c", src, "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{r.stderr[-6000:]}")

@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "common.h"
+#include "qgemm.h"
 
 namespace qraf_hip {
 
@@ -96,6 +97,7 @@ int qraf_hip_init(int device) {
     QH_CHECK_HIP(hipSetDevice(device));
     QH_TRY(ensure_init());
     QH_TRY(qgemm_kw_init());
+    QH_TRY(qgemm_wide_init());
     return attn_scratch_init(device);
 }
 

@@ -36,6 +36,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "qgemm.h"
 
 namespace qraf_hip {
 
@@ -1366,6 +1367,7 @@ struct QgPlan {
     bool pipe;  // qgemm_pipe_kernel (tile-major weights, batch tiles over 32 rows)
     int kwR, kwT;  // kwR > 0: qgemm_kw_kernel<FMT, kwR, kwT> (tile-major weights)
     int kxT;       // > 0: qgemm_kx_kernel<FMT, 3, kxT, 1> (tile-major weights)
+    int wide;      // > 0: form wide - 1 of qgemm_wide.hip (tile-major weights)
     int skG;    // > 0: stream-K over skG workgroups (pipelined kernel only); S = the slices a tile may need
     size_t ws_bytes;
 };
@@ -1507,8 +1509,68 @@ static bool kx_wanted(uint32_t dtype, int N, int K, int M) {
     return (M > 32 && M <= 64 && N >= 16384) || (M > 64 && dtype == DT_Q8_0 && K >= 8192);
 }
 
-static QgPlan qgemm_plan(uint32_t dtype, int N, int K, int M, size_t row_bytes, bool tiled) {
+// Whether the 32x32 kernel (qgemm_wide.hip) takes a tiled N x K product of M
+// rows, unless a tuning call forces an older form.  Both sides measured on
+// MI355X over 20-512 rows of the Qwen2.5-3B, SmolLM2 and head shapes (GEMM and
+// partial sums, graph-timed); it is the faster one (1.05-2.8x) except
+//   17-32 rows of Q8_0 (2048 x 2048 7.8 against 9.2 us, 22016 x 2048 24.1 against
+//   23.4) and of small Q4_0 products (2048 x 2048 7.9 against 8.5; 2560 x 2048 is
+//   8.8 against 7.9), where a workgroup's start and end are most of its time;
+//   more than 64 rows of the largest outputs (Q4_0 22016 x 2048 at 384 rows 90.8
+//   against 102.9 us, at 256 rows 65.4 against 57.0; Q8_0 11008 x 2048 at 384 rows
+//   65.5 against 70.4, at 256 rows 44.7 against 36.6; the 151936-row head at 128
+//   rows ties): several full rounds of workgroups, where the older kernels' two
+//   workgroups per CU hide each other's start and end.  The SwiGLU entry's other
+//   form below 256 rows is slower (Q8_0 at 203 rows 116.8 against 79.7).
+// The offsets of a 128-row chunk are 32-bit: N and K below 2^22.
+static bool wide_wanted(uint32_t dtype, int N, int K, int M, bool whole = false) {
+    if (g_qg_pipe || g_qg_kw || g_qg_mchunk || g_qg_waves || g_qg_splits || g_qg_sched == 1) return false;
+    if (M <= 16 || N >= (1 << 22) || K >= (1 << 22)) return false;
+    if (M <= 32) return dtype == DT_Q4_0 && (size_t)N * K > (size_t)4608 * 1024;
+    return M <= 64 || (whole && M < 256) || (size_t)M * N <= (size_t)(dtype == DT_Q8_0 ? 4 : 8) << 20;
+}
+
+// The wide kernel's form and split count: the least rounds of workgroups (one
+// per CU) x (iterations x us each + us to start and finish), plus the launch and
+// the traffic of the partial slices.  The us were fitted to each form's time
+// over K (MI355X: 256 rows of weights, one round, K = 4096 and 8192).
+static void wide_plan(QgPlan& p, uint32_t dtype, int N, int nb, int M, bool whole) {
+    static constexpr struct {
+        double it[2], fix;  // Q4_0, Q8_0
+    } T[QW_FORM_COUNT] = {{{1.60, 1.70}, 5.0}, {{1.00, 1.35}, 2.5}, {{1.15, 1.38}, 2.5}, {{0.79, 0.98}, 1.5}};
+    const int np = (nb + 1) / 2, cu = qg_cu_count();  // pairs of quant blocks
+    double best = 1e30;
+    for (int i = 0; i < QW_FORM_COUNT; i++) {
+        const QwTile t = qgemm_wide_tile(i);
+        const long long tiles = (long long)((N + t.nt - 1) / t.nt) * ((M + t.mt - 1) / t.mt);
+        for (int S = 1; S <= (whole ? 1 : 16); S++) {
+            const int pps = (np + S - 1) / S;
+            if ((np + pps - 1) / pps != S) continue;
+            const long long rounds = (tiles * S + cu - 1) / cu;
+            const double us = rounds * ((pps + t.wk - 1) / t.wk * T[i].it[dtype == DT_Q8_0] + T[i].fix) +
+                              (S > 1 ? 2.5 + (double)S * M * N * 2e-6 : 0.0);
+            if (us < best) {
+                best = us;
+                p.wide = i + 1;
+                p.bps = 2 * pps;
+                p.S = S;
+                p.ntiles = (N + t.nt - 1) / t.nt;
+                p.mchunks = (M + t.mt - 1) / t.mt;
+                p.MW = t.mt;
+                p.NW = t.nt;
+            }
+        }
+    }
+    p.ws_bytes = p.S > 1 ? (size_t)p.S * M * N * 4 : 0;
+}
+
+// wide: the 32x32 kernel may be the plan (the argmax epilogue exists in the pipelined one only)
+static QgPlan qgemm_plan(uint32_t dtype, int N, int K, int M, size_t row_bytes, bool tiled, bool wide = true) {
     QgPlan p{};
+    if (tiled && wide && wide_wanted(dtype, N, K, M)) {
+        wide_plan(p, dtype, N, K / 32, M, false);
+        return p;
+    }
     if (tiled && kx_wanted(dtype, N, K, M)) {
         kx_plan(p, N, K / 32, M, false);
         return p;
@@ -1680,12 +1742,17 @@ int set_qgemm_tuning(int waves, int splits, int pipe, int mchunk) {
 
 size_t qgemm_workspace_bytes(uint32_t dtype, int N, int K, int M, bool tiled) {
     if ((dtype != DT_Q8_0 && dtype != DT_Q4_0) || N <= 0 || K <= 0 || K % 32 || M <= 0) return 0;
-    return qgemm_plan(dtype, N, K, M, q_row_bytes(dtype, 32, K), tiled).ws_bytes;
+    // covers the plan with and without the 32x32 kernel: one allocation serves the
+    // product whichever form a later tuning call selects
+    const size_t rb = q_row_bytes(dtype, 32, K);
+    return std::max(qgemm_plan(dtype, N, K, M, rb, tiled).ws_bytes, qgemm_plan(dtype, N, K, M, rb, tiled, false).ws_bytes);
 }
 
 size_t qgemm_partials_bytes(uint32_t dtype, int N, int K, int M, bool tiled) {
     if ((dtype != DT_Q8_0 && dtype != DT_Q4_0) || N <= 0 || K <= 0 || K % 32 || M <= 0) return 0;
-    return (size_t)qgemm_plan(dtype, N, K, M, q_row_bytes(dtype, 32, K), tiled).S * M * N * 4;
+    const size_t rb = q_row_bytes(dtype, 32, K);
+    const int S = std::max(qgemm_plan(dtype, N, K, M, rb, tiled).S, qgemm_plan(dtype, N, K, M, rb, tiled, false).S);
+    return (size_t)S * M * N * 4;
 }
 
 int launch_split_bf16(const float* x, uint16_t* hi, uint16_t* lo, int M, int K, int op, float* xout, hipStream_t s,
@@ -1866,13 +1933,16 @@ int launch_qgemm(const void* W, uint32_t dtype, int bs, int N, int K, const uint
         } else {  // no (or too small a) workspace: one split
             p.S = 1;
             p.skG = 0;
-            const int unit = (p.kwR || p.kxT) ? 1 : (p.pipe ? 1 : 2) * p.KC;
+            const int unit = p.wide ? 2 : (p.kwR || p.kxT) ? 1 : (p.pipe ? 1 : 2) * p.KC;
             p.bps = (nb + unit - 1) / unit * unit;
         }
     }
     QH_REQUIRE(p.mchunks <= 65535, QRAF_HIP_ERR_INVALID, "qgemm: batch %d too large", M);
     const dim3 grid = p.skG > 0 ? dim3(p.skG, 1, 1) : dim3(p.ntiles, p.S, p.mchunks);
-    if (p.kxT) {
+    if (p.wide) {
+        QH_TRY(launch_qgemm_wide(p.wide - 1, W, dtype, N, K, xh, xl, M, part ? part : Y, part ? nullptr : add, p.S, p.bps,
+                                 nullptr, nullptr, s));
+    } else if (p.kxT) {
 #define QH_KX(F, T_)                                                                                          \
     hipLaunchKernelGGL((qgemm_kx_kernel<F, 3, T_, 1>), grid, dim3(256), 0, s, (const uint8_t*)W, N, nb, xh, xl, K, M, \
                        Y, add, p.bps, part, nullptr, nullptr)
@@ -1972,7 +2042,7 @@ size_t qgemm_argmax_keys_bytes(int N, int M) {
 // or the keys do not fit)
 static bool argmax_plan(uint32_t dtype, int N, int K, int M, size_t keys_bytes, QgPlan& p) {
     if ((dtype != DT_Q8_0 && dtype != DT_Q4_0) || K <= 0 || K % 32 || N <= 0 || M <= 0) return false;
-    p = qgemm_plan(dtype, N, K, M, q_row_bytes(dtype, 32, K), true);
+    p = qgemm_plan(dtype, N, K, M, q_row_bytes(dtype, 32, K), true, false);
     if (!p.pipe || p.kwR || p.kxT) return false;
     p.S = 1;  // complete sums in every workgroup
     p.skG = 0;
@@ -2018,6 +2088,11 @@ int launch_qgemm_silu(const void* Wt, uint32_t dtype, int N, int K, const uint16
     QH_REQUIRE(((((uintptr_t)Wt) | ((uintptr_t)xh) | ((uintptr_t)xl)) & 15) == 0, QRAF_HIP_ERR_INVALID,
                "qgemm silu: misaligned operands");
     const int nb = K / 32, KC = 2;
+    if (wide_wanted(dtype, N, K, M, true)) {
+        QgPlan p{};
+        wide_plan(p, dtype, N, nb, M, true);
+        return launch_qgemm_wide(p.wide - 1, Wt, dtype, N, K, xh, xl, M, nullptr, nullptr, 1, p.bps, act_hi, act_lo, s);
+    }
     if (g_qg_pipe == 3 ? M > 16 : (g_qg_pipe == 0 && g_qg_kw == 0 && M >= 256)) {
         QgPlan p{};
         kx_plan(p, N, nb, M, true);

@@ -509,3 +509,34 @@ def test_qgemm_tiled_argmax(hip, dt, case):
     assert np.array_equal(dtok.download(np.uint32, M), sentinel)  # not fused: tokens untouched
     for d in (dw, dx, dtl, dh, dl, keys, dtok):
         d.free()
+
+
+@pytest.mark.parametrize("dt", [po.Q8_0, po.Q4_0])
+@pytest.mark.parametrize("case", [
+    # N, K, M: one block and an odd count (half a pair at a group's end), fewer pairs than K groups, ragged rows
+    # and columns of each tile height (32, 64, 128 rows), splits with an odd tail
+    (64, 32, 33), (100, 96, 40), (33, 64, 64), (300, 416, 65), (1000, 2080, 129), (130, 2048, 203), (2050, 1056, 97),
+    (9000, 576, 20), (4100, 2048, 32), (12000, 2048, 200)], ids=lambda c: "x".join(map(str, c)))
+def test_qgemm_32x32_edges(hip, dt, case):
+    """The 32x32 kernel's tiles, K groups and splits at their edges, against the
+    oracle within the GEMM's bound, with a residual added in place; and a row
+    of NaN and one of infinities leave every other row as it was, bit for bit
+    (blocks past the end of a row or of a split belong to other rows)."""
+    N, K, M = case
+    rng = np.random.default_rng(3 * N + K + 7 * M + dt)
+    wq = po.quantize(dt, (rng.standard_normal(N * K) * 0.02).astype(np.float32))
+    X = rng.standard_normal((M, K)).astype(np.float32)
+    add = rng.standard_normal((M, N)).astype(np.float32)
+    print(f"qgemm 32x32 N={N} K={K} M={M} dt={dt}", flush=True)
+    Y, _, _ = run_gemm(hip, wq, dt, N, K, X, tiled=True, repeats=2)
+    check(Y, wq, dt, N, K, X)
+    Ya, _, _ = run_gemm(hip, wq, dt, N, K, X, add=add, in_place=True, tiled=True)
+    check(Ya, wq, dt, N, K, X, add)
+    bad = X.copy()
+    bad[M // 2, :] = np.nan
+    bad[M - 1, :] = np.inf
+    Yb, _, _ = run_gemm(hip, wq, dt, N, K, bad, tiled=True)
+    keep = np.ones(M, bool)
+    keep[[M // 2, M - 1]] = False
+    assert np.array_equal(Yb[keep].view(np.uint32), Y[keep].view(np.uint32))
+    assert not np.isfinite(Yb[~keep]).any()
