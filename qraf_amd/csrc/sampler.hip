@@ -17,6 +17,10 @@
 //      LDS by (p descending, index ascending).  The reference's std::sort
 //      leaves the order of equal p unspecified; this order is one of its
 //      possible results.
+//      Rows of at least SUB_MIN logits with a small cutoff skip 2: one read of the
+//      row leaves each thread the largest of its 4 sub-ranges; a value that cutoff
+//      of those 4096 maxima reach bounds the cutoff-th largest p from below, and
+//      only sub-ranges whose maximum reaches it are read again, to gather.
 //   4. The reference's arithmetic on the sorted candidates in its order:
 //      exp(p - max) and the divisions elementwise (all threads), the
 //      sequential sums, top-p prefix, renormalisation and the cumulative sum
@@ -55,6 +59,11 @@ namespace qraf_hip {
 constexpr int CAND_CAP = 4096;  // candidates gathered and sorted in LDS at most
 
 constexpr int SNT = 1024;  // threads per row (16 waves)
+
+// the sub-range maxima path: sub-ranges per thread, the shortest row (every
+// sub-range then has an element), the largest cutoff (4096 maxima bound it
+// within a few per cent)
+constexpr int NSUB = 4, SUB_MIN = 4 * NSUB * SNT + 64, SUB_CUT = 512;
 
 // Row loops: each thread reads 4 float4 (16 logits) before using any, so a
 // workgroup has 16K logits in flight per round trip; f(i, value) is called
@@ -299,6 +308,60 @@ __device__ uint32_t sorted_pairs_pick(float* pv, const int* iv, int n, float top
     return (uint32_t)iv[at < 0 ? m - 1 : at];
 }
 
+// Sorting and the reference's loops (sampler.cpp:79-127) for n <= 64 gathered
+// pairs, of which the first nc after sorting are the candidates: one wave, a
+// pair per lane, the same additions and divisions in the same order as the
+// workgroup's code below.
+__device__ __forceinline__ void out_wave(const float* cval, const int* cidx, int n, int nc, float top_p, float r,
+                                         uint32_t* out) {
+    const int lane = threadIdx.x & 63;
+    float p = lane < n ? cval[lane] : -INFINITY;
+    int ix = lane < n ? cidx[lane] : 0x7FFFFFFF;
+#pragma unroll
+    for (int k = 2; k <= 64; k <<= 1)
+#pragma unroll
+        for (int j = k >> 1; j > 0; j >>= 1) {
+            const float op = __shfl_xor(p, j);
+            const int oi = __shfl_xor(ix, j);
+            const bool first = p > op || (p == op && ix < oi);  // p descending, index ascending
+            const bool want = ((lane & j) == 0) == ((lane & k) == 0);
+            if (first != want) {
+                p = op;
+                ix = oi;
+            }
+        }
+    auto at = [](float v, int i) {  // lane i's value (i uniform)
+        return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), i));
+    };
+    float e = expf(p - at(p, 0));
+    float sum = 0.f;
+    for (int i = 0; i < nc; i++) sum += at(e, i);
+    e /= sum;
+    int m = nc;
+    if (top_p > 0.f && top_p < 1.f) {
+        float cs = 0.f;  // also the nucleus' sum: the same additions
+        for (int i = 0; i < nc; i++) {
+            cs += at(e, i);
+            if (cs >= top_p) {
+                m = i + 1;
+                break;
+            }
+        }
+        if (lane < m) e /= cs;
+    }
+    float cs = 0.f;
+    int pick = m - 1;
+    for (int i = 0; i < m; i++) {
+        cs += at(e, i);
+        if (r <= cs) {
+            pick = i;
+            break;
+        }
+    }
+    const uint32_t token = (uint32_t)__builtin_amdgcn_readlane(ix, pick);
+    if (lane == 0) *out = token;
+}
+
 __global__ __launch_bounds__(SNT) void sample_rows_kernel(const float* __restrict__ logits, int V, float T, int cutoff,
                                                           float top_p, const float* __restrict__ uniforms,
                                                           uint32_t* __restrict__ out, float* __restrict__ sort_ws) {
@@ -361,6 +424,7 @@ __global__ __launch_bounds__(SNT) void sample_rows_kernel(const float* __restric
     __shared__ uint32_t s_last;  // trunc: the reference's last sorted token
     int nsort = cutoff;
     bool fast = cutoff == V;  // every token a candidate
+    bool gathered = false;    // the candidates are in cval / cidx
     float t = -INFINITY;
     // the row's sort storage: pairs (pa, ia), the radix sort's other buffer (pb, ib)
     float* pa = sort_ws + (size_t)row * 4 * V;
@@ -426,11 +490,134 @@ __global__ __launch_bounds__(SNT) void sample_rows_kernel(const float* __restric
         fast = !big;  // gather p >= t below, or sort every pair
     }
 
+    // ---- one read of the row and a search among sub-range maxima (see the file
+    // comment).  Bound by the row's bytes (one workgroup per row; the search passes
+    // below read the row once each): MI355X, 128 rows x 151936, top-k 40, top-p 0.9:
+    // 114 -> 28 us (77.8 MB read once: 15 us at the rate of a large copy).  Left to the searches below: maxima that are not finite
+    // (masked rows) and more than CAND_CAP values at the bound.
+    if (!fast && !big && (V & 3) == 0 && V >= SUB_MIN && cutoff <= SUB_CUT) {
+        const float4* l4 = (const float4*)l;
+        const int V4 = V >> 2, Q = (V4 + NSUB - 1) / NSUB;  // float4s per sub-range
+        float mx[NSUB];
+#pragma unroll
+        for (int q = 0; q < NSUB; q++) {
+            const int b0 = q * Q + tid, b1 = min(V4, (q + 1) * Q);
+            float m0 = -INFINITY, m1 = -INFINITY;
+            for (int base = b0; base < b1; base += SNT * 5) {
+                float4 v[5];
+#pragma unroll
+                for (int u = 0; u < 5; u++) v[u] = l4[base + SNT * u < b1 ? base + SNT * u : base];  // past the end: its own again
+#pragma unroll
+                for (int u = 0; u < 5; u++) {
+                    m0 = fmaxf(fmaxf(m0, v[u].x), v[u].y);
+                    m1 = fmaxf(fmaxf(m1, v[u].z), v[u].w);
+                }
+            }
+            mx[q] = b0 < b1 ? fmaxf(m0, m1) : -INFINITY;
+        }
+        // the row's largest value and the smallest maximum
+        float hi = fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3])), lo = fminf(fminf(mx[0], mx[1]), fminf(mx[2], mx[3]));
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) {
+            hi = fmaxf(hi, __shfl_xor(hi, o));
+            lo = fminf(lo, __shfl_xor(lo, o));
+        }
+        if ((tid & 63) == 0) {
+            s_red[0][tid >> 6] = hi;
+            s_red[1][tid >> 6] = lo;
+        }
+        __shared__ int s_sub[3][8];  // counts of a search pass; the pass after next's are cleared meanwhile
+        if (tid < 24) s_sub[tid >> 3][tid & 7] = 0;
+        if (tid == 0) s_n = 0;
+        __syncthreads();
+        for (int w = 0; w < NW; w++) {
+            hi = fmaxf(hi, s_red[0][w]);
+            lo = fminf(lo, s_red[1][w]);
+        }
+        __syncthreads();  // s_red may be written again
+        if (lo > -INFINITY && hi < INFINITY) {
+            // #{maxima >= lo} = clo >= cutoff throughout
+            int clo = NSUB * SNT;
+            const int target = cutoff + (cutoff >> 2) + 8;
+            for (int pass = 0; pass < 16 && clo > target && lo < hi; pass++) {
+                float th[8];
+                int mine = 0;
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    th[j] = lo + (hi - lo) * ((float)(j + 1) / 9.0f);
+                    int c = 0;
+#pragma unroll
+                    for (int q = 0; q < NSUB; q++) c += __popcll(__ballot(mx[q] >= th[j]));
+                    mine = (tid & 63) == j ? c : mine;
+                }
+                if ((tid & 63) < 8 && mine) atomicAdd(&s_sub[pass % 3][tid & 63], mine);
+                __syncthreads();
+                int c[8];
+#pragma unroll
+                for (int j = 0; j < 8; j++) c[j] = s_sub[pass % 3][j];
+                if (tid < 8) s_sub[(pass + 2) % 3][tid] = 0;  // last read before this pass's barrier
+                float nlo = lo, nhi = hi;
+                int cb = clo;
+#pragma unroll
+                for (int j = 0; j < 8; j++)
+                    if (c[j] >= cutoff) {
+                        nlo = th[j];
+                        cb = c[j];
+                        nhi = j < 7 ? th[j + 1] : hi;
+                    }
+                if (c[0] < cutoff) nhi = th[0];
+                if (!(nlo > lo || nhi < hi)) break;  // values too close together
+                lo = nlo;
+                hi = nhi;
+                clo = cb;
+            }
+            // every p at or above the bound's: p = v / T may round several v to one p, so
+            // values just below the bound are looked at too (the margin is 2^3 roundings
+            // and, for a subnormal p, as many of its steps)
+            const float pt = lo / T, tg = (float)((double)lo - fabs((double)lo) * 0x1p-20 - (double)T * 1e-37);
+#pragma unroll
+            for (int q = 0; q < NSUB; q++) {
+                if (!(mx[q] >= tg)) continue;
+                const int b1 = min(V4, (q + 1) * Q);
+                for (int base = q * Q + tid; base < b1; base += SNT * 5) {
+                    float4 v[5];
+#pragma unroll
+                    for (int u = 0; u < 5; u++) v[u] = l4[base + SNT * u < b1 ? base + SNT * u : base];
+#pragma unroll
+                    for (int u = 0; u < 5; u++) {
+                        const float x[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+#pragma unroll
+                        for (int e = 0; e < 4; e++)
+                            if (base + SNT * u < b1 && x[e] >= tg) {
+                                const float p = x[e] / T;
+                                if (p >= pt) {
+                                    const int k = atomicAdd(&s_n, 1);
+                                    if (k < CAND_CAP) {
+                                        cval[k] = p;
+                                        cidx[k] = 4 * (base + SNT * u) + e;
+                                    }
+                                }
+                            }
+                    }
+                }
+            }
+            __syncthreads();
+            gathered = s_n <= CAND_CAP;
+            if (gathered) nsort = s_n;
+            __syncthreads();  // s_n may be written again
+        }
+    }
+    if (gathered && nsort <= 64) {
+        // one wave: the candidates in its lanes, the sequential sums by lane reads
+        if (tid < 64) out_wave(cval, cidx, nsort, cutoff, top_p, uniforms[row], &out[row]);
+        return;
+    }
+
     // ---- fast path: a threshold t with cutoff <= #{p >= t} <= CAND_CAP, by an
     // 8-way search between the row's smallest and largest p; then every
     // p >= t is gathered and sorted.  The sort makes the result independent
     // of the gather order, and equal to the radix path's.
-    if (!fast && !big) {
+    if (!fast && !big && !gathered) {
         float mx = -INFINITY, mn = INFINITY;
         for_row(l, V, tid, [&](int, float v) {
             const float p = v / T;
@@ -499,7 +686,9 @@ __global__ __launch_bounds__(SNT) void sample_rows_kernel(const float* __restric
             }
         }
     }
-    if (fast) {
+    if (gathered) {
+        // cval / cidx hold the nsort candidates
+    } else if (fast) {
         if (tid == 0) s_n = 0;
         __syncthreads();
         for_row(l, V, tid, [&](int i, float v) {
@@ -637,31 +826,37 @@ __global__ __launch_bounds__(SNT) void sample_rows_kernel(const float* __restric
     __syncthreads();
     for (int i = tid; i < nc; i += SNT) cval[i] = expf(cval[i] - max_val);
     __syncthreads();
-    if (tid == 0) {
-        float sum = 0.f;
-        for (int i = 0; i < nc; i++) sum += cval[i];
-        s_sum = sum;
+    // the sequential sums: one wave, 64 terms at a time in its lanes (a thread
+    // reading LDS term by term waits a load's latency for each); stops at the
+    // first sum for which reach(sum) holds and returns its index, m if none
+    auto scan = [&](int m, float& cs, auto&& reach) {
+        cs = 0.f;
+        for (int c0 = 0; c0 < m; c0 += 64) {
+            const int v = __builtin_bit_cast(int, c0 + tid < m ? cval[c0 + tid] : 0.f);
+            for (int i = 0; i < min(64, m - c0); i++) {
+                cs += __builtin_bit_cast(float, __builtin_amdgcn_readlane(v, i));
+                if (reach(cs)) return c0 + i;
+            }
+        }
+        return m;
+    };
+    if (tid < 64) {
+        float cs;
+        scan(nc, cs, [](float) { return false; });
+        if (tid == 0) s_sum = cs;
     }
     __syncthreads();
     const float sum = s_sum;
     for (int i = tid; i < nc; i += SNT) cval[i] /= sum;
     __syncthreads();
     const bool topp = top_p > 0.f && top_p < 1.f;
-    if (topp && tid == 0) {
-        float cs = 0.f;
-        int nucleus = -1;  // -1: the prefix never reaches top_p (the whole list)
-        for (int i = 0; i < nc; i++) {
-            cs += cval[i];
-            if (cs >= top_p) {
-                nucleus = i + 1;
-                break;
-            }
+    if (topp && tid < 64) {
+        float cs;  // the nucleus' sum is the same additions up to its last term
+        const int i = scan(nc, cs, [&](float c) { return c >= top_p; });
+        if (tid == 0) {
+            s_sum = cs;
+            s_nucleus = i < nc ? i + 1 : -1;  // -1: the prefix never reaches top_p (the whole list)
         }
-        const int m = nucleus < 0 ? nc : nucleus;
-        float ns = 0.f;
-        for (int i = 0; i < m; i++) ns += cval[i];
-        s_sum = ns;
-        s_nucleus = nucleus;
     }
     __syncthreads();
     int nucleus = -1;
@@ -672,21 +867,15 @@ __global__ __launch_bounds__(SNT) void sample_rows_kernel(const float* __restric
         for (int i = tid; i < m; i += SNT) cval[i] /= ns;
         __syncthreads();
     }
-    if (tid == 0) {
+    if (tid < 64) {
         const int n = nucleus < 0 ? nc : nucleus;
         const float r = uniforms[row];
-        float cs = 0.f;
+        float cs;
+        const int i = scan(n, cs, [&](float c) { return r <= c; });
         // fallback: the reference's last candidate; with an absorbed tail and
         // no nucleus that is its last sorted token of the whole vocabulary
-        uint32_t pick = trunc && nucleus < 0 ? s_last : (uint32_t)cidx[n - 1];
-        for (int i = 0; i < n; i++) {
-            cs += cval[i];
-            if (r <= cs) {
-                pick = (uint32_t)cidx[i];
-                break;
-            }
-        }
-        out[row] = pick;
+        if (tid == 0)
+            out[row] = i < n ? (uint32_t)cidx[i] : trunc && nucleus < 0 ? s_last : (uint32_t)cidx[n - 1];
     }
 }
 

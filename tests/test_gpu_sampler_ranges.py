@@ -1,0 +1,67 @@
+"""Device sampler at the edges of its sub-range maxima path, against
+Sampler::sample (sampler.cpp:57-128) restated in numpy float32: the sorted
+candidates by (p descending, index ascending), exp(p - max), the sequential
+sums in order, top-p, and the cumulative sum against the uniform.  A uniform
+that lands within 1e-5 of a cumulative boundary is moved to the middle of its
+interval (device expf against numpy's differs in the last place)."""
+import numpy as np
+import pytest
+
+from tests.test_gpu_sampler import device_sample
+
+pytestmark = pytest.mark.gpu
+
+
+def candidates(l, T, k, top_p):
+    p = (l / np.float32(T)).astype(np.float32)
+    o = np.lexsort((np.arange(l.size), -p))[:k]
+    e = np.exp(p[o] - p[o[0]]).astype(np.float32)
+    e = (e / np.cumsum(e, dtype=np.float32)[-1]).astype(np.float32)
+    if 0.0 < top_p < 1.0:
+        cs = np.cumsum(e, dtype=np.float32)
+        m = int(np.argmax(cs >= np.float32(top_p))) + 1 if (cs >= np.float32(top_p)).any() else k
+        o, e = o[:m], (e[:m] / cs[m - 1]).astype(np.float32)
+    return o, np.cumsum(e, dtype=np.float32)
+
+
+def pick(o, cs, r):
+    hit = np.nonzero(np.float32(r) <= cs)[0]
+    return o[hit[0]] if hit.size else o[-1]
+
+
+@pytest.mark.parametrize("V", [16380, 16448, 16452, 20004, 151936])
+@pytest.mark.parametrize("k", [1, 40, 64, 65, 512, 513])
+def test_sampling_with_sub_range_maxima(hip, V, k):
+    rng = np.random.default_rng(V + k)
+    rows = []
+    q = (V // 4 + 3) // 4  # float4s of a sub-range
+    for kind in range(6):
+        l = (rng.standard_normal(V) * 2).astype(np.float32)
+        if kind == 1:  # the row's largest values at the sub-ranges' ends
+            for s in range(1, 5):
+                l[min(V, 4 * q * s) - 4:min(V, 4 * q * s)] = 20 + rng.random(4)
+        elif kind == 2:  # many equal values around the cutoff
+            l = np.round(l * 4) / 4
+        elif kind == 3:  # the candidates all in one thread's reach
+            l[4 * np.arange(8) * 1024 % (V - 4)] = 15 + np.arange(8)
+        elif kind == 4:  # a masked row (left to the search over the row)
+            l[::3] = -np.inf
+        elif kind == 5:  # distinct logits that round to one p
+            l[100:100 + 64] = np.nextafter(np.float32(9), np.float32(10)) + np.float32(1e-6) * np.arange(64)
+        rows.append(l.astype(np.float32))
+    L = np.stack(rows)
+    for T, top_p in ((0.8, 0.9), (1.7, 1.0), (3.0, 0.5)):
+        want, uni = [], []
+        for l in rows:
+            o, cs = candidates(l, T, k, top_p)
+            r = np.float32(rng.random())
+            j = int(np.searchsorted(cs, r))
+            if np.abs(cs - r).min() < 1e-5:
+                lo = cs[j - 1] if j > 0 else np.float32(0)
+                r = np.float32((float(lo) + float(cs[min(j, cs.size - 1)])) / 2)
+            clear = np.abs(cs - r).min() >= 1e-6  # else several boundaries in one place: any of their tokens
+            want.append(pick(o, cs, r) if clear else None)
+            uni.append(r)
+        got, _ = device_sample(hip, L, (T, k, top_p, 1.0), uniforms=np.array(uni, np.float32))
+        for kind, (g, w) in enumerate(zip(got, want)):
+            assert w is None or g == w, f"V={V} k={k} T={T} top_p={top_p} kind={kind}: {g} against {w}"
