@@ -98,6 +98,7 @@ int qraf_hip_init(int device) {
     QH_TRY(ensure_init());
     QH_TRY(qgemm_kw_init());
     QH_TRY(qgemm_wide_init());
+    QH_TRY(attention_init());
     return attn_scratch_init(device);
 }
 

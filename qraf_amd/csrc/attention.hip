@@ -19,6 +19,8 @@
 // chunks of CH = 256 positions; one workgroup handles one (sequence, chunk)
 // item for one KV head and all H/Hkv query heads that share it (GQA).  The
 // grid has ceil(max_ctx / CH) items per sequence (item = s * that + chunk);
+// with up to 1,024 positions a workgroup may hold the whole context
+// (chunk_waves: 8, 12 or 16 waves, no merge);
 // a workgroup whose chunk starts at or past its sequence's device-resident
 // context length exits at once, so the lengths can change on the device
 // between launches with no host round trip.  Sequences with several chunks
@@ -104,12 +106,13 @@ __device__ __forceinline__ void attn_store(const AttnArgs& a, size_t i, float v)
 
 // Item -> (sequence, chunk): item = s * chunks_per_seq + chunk.  Returns
 // false when the chunk starts at or past the sequence's context.
+template <int CH>
 __device__ __forceinline__ bool attn_item(const AttnArgs& a, int& s, int& chunk, int& nchunks, int& ctx) {
-    const int per = (a.max_ctx + ACH - 1) / ACH;
+    const int per = (a.max_ctx + CH - 1) / CH;
     s = blockIdx.x / per;
     chunk = blockIdx.x - s * per;
     ctx = min(a.ctx[s], a.max_ctx);
-    nchunks = (ctx + ACH - 1) / ACH;
+    nchunks = (ctx + CH - 1) / CH;
     return chunk < nchunks;
 }
 
@@ -305,8 +308,8 @@ __global__ __launch_bounds__(ACH) void attn_decode_kernel(AttnArgs a) {
 
 // ---------------------------------------------------------------------------
 // Matrix-core decode attention for fp16 pages (see the file comment).  One
-// workgroup = one (sequence, ACH-position chunk, KV head); wave w takes the
-// chunk's positions 64w .. 64w+63 as four 16-position tiles.
+// workgroup = one (sequence, chunk of 64 NW positions, KV head); wave w takes
+// the chunk's positions 64w .. 64w+63 as four 16-position tiles.
 //
 // q.K^T, per tile: A = K (lane: position l%16, 8 dimensions), B = q^T (lane:
 // head l%16, the same 8 dimensions), D[position][head]; heads >= G are zero
@@ -443,13 +446,15 @@ __device__ __forceinline__ f16x8 i8x8_to_f16x8(uint32_t w0, uint32_t w1) {
     return __builtin_bit_cast(f16x8, make_uint4(a.x, a.y, b.x, b.y));
 }
 
-// 4 workgroups per CU (at most 128 VGPRs): the K and V loads of one wave
-// already cover its own latency, more resident workgroups cover the
-// prologue and epilogue of the others
-template <int HD, int KV, bool UPG>
-__global__ __launch_bounds__(ACH, 4) void attn_mfma_kernel(AttnArgs a, int G) {
+// 16 waves per CU (at most 128 VGPRs; 12-wave workgroups, which take the CU
+// alone, 168): the K and V loads of one wave already cover its own latency,
+// more resident waves cover the prologue and epilogue of the others.  NW as
+// chosen by chunk_waves; the waves past the context hold no partial outputs
+template <int HD, int KV, bool UPG, int NW>
+__global__ __launch_bounds__(64 * NW, NW == 12 ? 3 : 4) void attn_mfma_kernel(AttnArgs a, int G) {
     static_assert(HD == 64 || HD == 128, "head_dim 64 or 128");
     constexpr bool I8 = KV == KV_I8, F32 = KV == KV_F32;
+    constexpr int CH = 64 * NW, HJ = (16 + NW - 1) / NW;  // positions, q heads staged per wave
     constexpr int KK = HD / 32;  // MFMA k-steps per score tile
     // q.K^T k-step kk, lane group s = l/16 covers 8 dimensions starting at
     // kdim(kk, s).  fp16: 8*(4kk+s), so the 4 groups of one step read 64
@@ -464,9 +469,9 @@ __global__ __launch_bounds__(ACH, 4) void attn_mfma_kernel(AttnArgs a, int G) {
     _Float16(*s_q)[16][QS] = (_Float16(*)[16][QS])s_qbuf;
     float(*s_qf)[HD + 4] = (float(*)[HD + 4])s_qbuf;
     __shared__ float s_qs[16];
-    __shared__ float s_m[4][16], s_l[4][16];
-    __shared__ __align__(16) float s_kvs[2][4][64];  // int8: K, V scale of position pw + lane, per wave
-    extern __shared__ __align__(16) float s_odyn[];  // [4][G][HD]: the waves' partial outputs
+    __shared__ float s_m[NW][16], s_l[NW][16];
+    __shared__ __align__(16) float s_kvs[2][NW][64];  // int8: K, V scale of position pw + lane, per wave
+    extern __shared__ __align__(16) float s_odyn[];  // [NW][G][HD]: the waves' partial outputs
     float(*s_o)[HD] = (float(*)[HD])s_odyn;  // s_o[wave * G + head][dim]
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -475,10 +480,10 @@ __global__ __launch_bounds__(ACH, 4) void attn_mfma_kernel(AttnArgs a, int G) {
     const int item = blockIdx.x;
     int s, chunk, nchunks;
     int ctx;
-    if (!attn_item(a, s, chunk, nchunks, ctx)) return;
+    if (!attn_item<CH>(a, s, chunk, nchunks, ctx)) return;
     const int ps = a.page_size, psl = a.ps_log2, psm = ps - 1;  // page_size is a power of two here
     const int32_t* ptab = a.page_table + (size_t)s * a.max_pages;
-    const int pw = chunk * ACH + 64 * wave;  // first position of this wave
+    const int pw = chunk * CH + 64 * wave;  // first position of this wave
     const bool active = pw < ctx;            // wave-uniform
 
     // Every global read that does not depend on another is requested before
@@ -486,10 +491,10 @@ __global__ __launch_bounds__(ACH, 4) void attn_mfma_kernel(AttnArgs a, int G) {
     // (page ids known) the K rows, V runs and scales before q is staged, so
     // the staging and its barrier overlap those loads.
     constexpr int PER = HD / 64;
-    float qv[4][PER];  // q of head wave + 4j, dimensions lane + 64i
+    float qv[HJ][PER];  // q of head wave + NW j, dimensions lane + 64i
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int h = wave + 4 * j;
+    for (int j = 0; j < HJ; j++) {
+        const int h = wave + NW * j;
 #pragma unroll
         for (int i = 0; i < PER; i++)
             qv[j][i] = h < G ? a.q[((size_t)s * a.H + kvh * G + h) * HD + lane + 64 * i] : 0.f;
@@ -589,16 +594,18 @@ __global__ __launch_bounds__(ACH, 4) void attn_mfma_kernel(AttnArgs a, int G) {
     // then carries 22 bits of every element that matters at fp32 precision
     if constexpr (F32) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int h = wave + 4 * j;
+        for (int j = 0; j < HJ; j++) {
+            const int h = wave + NW * j;
+            if (16 % NW != 0 && h >= 16) break;
 #pragma unroll
             for (int i = 0; i < PER; i++) s_qf[h][lane + 64 * i] = qv[j][i];
             if (lane == 0) s_qs[h] = a.scale;  // attention.cpp:134: dot * scale
         }
     } else {
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int h = wave + 4 * j;
+    for (int j = 0; j < HJ; j++) {
+        const int h = wave + NW * j;
+        if (16 % NW != 0 && h >= 16) break;
         float* v = qv[j];
         float mx = 0.f;
 #pragma unroll
@@ -693,7 +700,9 @@ __global__ __launch_bounds__(ACH, 4) void attn_mfma_kernel(AttnArgs a, int G) {
     mloc = fmaxf(mloc, __shfl_xor(mloc, 32));
     if (seg == 0) s_m[wave][l16] = mloc;
     __syncthreads();
-    const float m = fmaxf(fmaxf(s_m[0][l16], s_m[1][l16]), fmaxf(s_m[2][l16], s_m[3][l16]));
+    float m = s_m[0][l16];
+#pragma unroll
+    for (int v = 1; v < NW; v++) m = fmaxf(m, s_m[v][l16]);
     float lsum = 0.f;
 #pragma unroll
     for (int t = 0; t < 4; t++)
@@ -781,13 +790,13 @@ __global__ __launch_bounds__(ACH, 4) void attn_mfma_kernel(AttnArgs a, int G) {
         pv(1, va1, vb1);
     }
 
-    // ---- combine the 4 waves: o[d][r] = O[head 4seg+r][dim 16d+l16]
+    // ---- combine the waves with positions: o[d][r] = O[head 4seg+r][dim 16d+l16]
     // (f32 pages: dim dvf(l16, d), four consecutive dims per float4)
     if constexpr (F32) {
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             const int h = 4 * seg + r;
-            if (h < G)
+            if (h < G && (NW == 4 || active))
 #pragma unroll
                 for (int i = 0; i < DT / 4; i++)
                     *(float4*)&s_o[wave * G + h][dvf(l16, 4 * i)] =
@@ -799,29 +808,50 @@ __global__ __launch_bounds__(ACH, 4) void attn_mfma_kernel(AttnArgs a, int G) {
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             const int h = 4 * seg + r;
-            if (h < G) s_o[wave * G + h][16 * d + l16] = o[d][r] * ounit;
+            if (h < G && (NW == 4 || active)) s_o[wave * G + h][16 * d + l16] = o[d][r] * ounit;
         }
     }
     __syncthreads();
+    const int na = NW == 4 ? 4 : min(NW, (ctx - chunk * CH + 63) >> 6);  // waves with positions
+    auto osum = [&](int h, int dd) {
+        if constexpr (NW == 4) {
+            return (s_o[h][dd] + s_o[G + h][dd]) + (s_o[2 * G + h][dd] + s_o[3 * G + h][dd]);
+        } else {
+            float x = s_o[h][dd];
+            for (int v = 1; v < na; v++) x += s_o[v * G + h][dd];
+            return x;
+        }
+    };
+    auto lsum_of = [&](int h) {
+        if constexpr (NW == 4) {
+            return (s_l[0][h] + s_l[1][h]) + (s_l[2][h] + s_l[3][h]);
+        } else {
+            float x = s_l[0][h];
+#pragma unroll
+            for (int v = 1; v < NW; v++) x += s_l[v][h];  // 0 for a wave without positions
+            return x;
+        }
+    };
     const size_t hbase = (size_t)s * a.H + kvh * G;
     if (nchunks == 1) {
-        for (int i = tid; i < G * HD; i += ACH) {
+        for (int i = tid; i < G * HD; i += CH) {
             const int h = i / HD, dd = i % HD;
-            const float O = (s_o[h][dd] + s_o[G + h][dd]) + (s_o[2 * G + h][dd] + s_o[3 * G + h][dd]);
-            const float L = (s_l[0][h] + s_l[1][h]) + (s_l[2][h] + s_l[3][h]);
-            attn_store(a, (hbase + h) * HD + dd, O / L);
+            attn_store(a, (hbase + h) * HD + dd, osum(h, dd) / lsum_of(h));
         }
         return;
     }
     // ---- multi-chunk: publish (max, sum, unnormalised output) for attn_merge_kernel
     const size_t ibase = (size_t)item * a.H + kvh * G;
-    for (int i = tid; i < G * HD; i += ACH) {
+    for (int i = tid; i < G * HD; i += CH) {
         const int h = i / HD, dd = i % HD;
-        a.part_o[(ibase + h) * HD + dd] = (s_o[h][dd] + s_o[G + h][dd]) + (s_o[2 * G + h][dd] + s_o[3 * G + h][dd]);
+        a.part_o[(ibase + h) * HD + dd] = osum(h, dd);
     }
     if (tid < G) {
-        a.part_ml[(ibase + tid) * 2 + 0] = fmaxf(fmaxf(s_m[0][tid], s_m[1][tid]), fmaxf(s_m[2][tid], s_m[3][tid]));
-        a.part_ml[(ibase + tid) * 2 + 1] = (s_l[0][tid] + s_l[1][tid]) + (s_l[2][tid] + s_l[3][tid]);
+        float M = s_m[0][tid];
+#pragma unroll
+        for (int v = 1; v < NW; v++) M = fmaxf(M, s_m[v][tid]);
+        a.part_ml[(ibase + tid) * 2 + 0] = M;
+        a.part_ml[(ibase + tid) * 2 + 1] = lsum_of(tid);
     }
 }
 
@@ -1423,12 +1453,50 @@ size_t attn_workspace_bytes(int n, int H, int Hkv, int hd, int max_ctx) {
            slots * H * hd * 4;
 }
 
-// 0: automatic (the balanced split when the chunk grid would need more than
+// 0: automatic (the balanced split when a grid of 256-position chunks would need more than
 // one round of resident workgroups, 4 per CU x 256 CUs, at the host-known
 // bound n x ceil(max_ctx / 256); below that the chunk grid, whose per-chunk
 // workgroups carry no share bookkeeping), 1: chunk grid, 2: balanced split,
 // 3: the plain fp32 VALU kernel for f32 and fp16 pages (int8 pages: automatic)
 static int g_attn_form = 0;
+
+// Waves per workgroup of the matrix-core chunk grid, one 64-position tile
+// each.  Contexts that may pass one 256-position chunk get a workgroup of 8,
+// 12 or 16 waves where that holds the whole context: no partials and no merge
+// launch (4-5 us behind a kernel of 6-30 us).  8 waves (up to 512 positions):
+// always; two such workgroups share a CU, so the chip fills as before (128
+// sequences x 2 KV heads x 8 heads, ctx 150-300: f16 18.7 -> 12.8 us, f32
+// 28.6 -> 22.9; one sequence of 512: 11.4 -> 10.6, 16.7 -> 16.3; 128 x 8 KV
+// heads of 512: 55.8 -> 47.5, 91.8 -> 84.1).  12 and 16 waves (768, 1,024
+// positions) take a whole CU and are the slower form where they leave CUs idle
+// that more workgroups would use, or need a second round: 12 waves from half
+// of the 256 CUs to all of them (192 workgroups 19.7 -> 17.0 us f16, 32.7 ->
+// 30.7 f32; 128: 16.5 -> 16.0, 27.8 -> 28.4; 272: 23.3 -> 27.8, 38.9 -> 49.7),
+// 16 waves from three quarters (224 workgroups 25.2 -> 20.2, 42.1 -> 39.1;
+// 192: 21.6 -> 21.5, 36.4 -> 38.2; 272: 31.0 -> 34.1, 55.0 -> 58.5).
+static int chunk_waves(int n, int Hkv, int max_ctx) {
+    const int wgs = n * Hkv;
+    if (g_attn_form == 1 || max_ctx <= ACH || max_ctx > 1024) return 4;
+    if (max_ctx <= 512) return 8;
+    if (max_ctx <= 768) return wgs > 128 && wgs <= 256 ? 12 : 4;
+    return wgs > 192 && wgs <= 256 ? 16 : 4;
+}
+
+// Wide workgroups hold up to 16 waves x 16 heads x 128 dimensions of partial
+// outputs in dynamic LDS (128 KB): the limit is raised once, at start-up
+int attention_init() {
+#define QH_ATTN_LDS1(HDv, KINDv, NWv, U)                                                    \
+    QH_CHECK_HIP(hipFuncSetAttribute((const void*)attn_mfma_kernel<HDv, KINDv, U, NWv>,     \
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, NWv * 16 * HDv * 4));
+#define QH_ATTN_LDS(HDv, KINDv, NWv) QH_ATTN_LDS1(HDv, KINDv, NWv, true) QH_ATTN_LDS1(HDv, KINDv, NWv, false)
+#define QH_ATTN_LDSN(HDv, KINDv) QH_ATTN_LDS(HDv, KINDv, 8) QH_ATTN_LDS(HDv, KINDv, 12) QH_ATTN_LDS(HDv, KINDv, 16)
+    QH_ATTN_LDSN(128, KV_F16) QH_ATTN_LDSN(64, KV_F16) QH_ATTN_LDSN(128, KV_I8)
+    QH_ATTN_LDSN(64, KV_I8) QH_ATTN_LDSN(128, KV_F32) QH_ATTN_LDSN(64, KV_F32)
+#undef QH_ATTN_LDSN
+#undef QH_ATTN_LDS
+#undef QH_ATTN_LDS1
+    return QRAF_HIP_OK;
+}
 
 int launch_attention(const float* q, const void* kc, const void* vc, uint32_t kv_dtype, const int32_t* page_table,
                      int max_pages, const int32_t* ctx, int n, int H, int Hkv, int hd, int page_size, float scale,
@@ -1488,29 +1556,38 @@ int launch_attention(const float* q, const void* kc, const void* vc, uint32_t kv
     const bool single_f32 = kv_dtype == DT_F32 && hd == 64 && n == 1 && max_ctx <= ACH && g_attn_form == 0;
     const bool valu = !mfma_shape || (g_attn_form == 3 && kv_dtype != DT_I8) || single_f32;
     const bool split = !valu && (g_attn_form == 2 || (g_attn_form != 1 && items > 1024));
+    const int nw = valu || split ? 4 : chunk_waves(n, Hkv, max_ctx);
     if (valu) {  // the plain fp32 VALU kernel
         if (kv_dtype == DT_F32) QH_TRY(launch_attn_t<float>(a, hd, G, items, st));
         else QH_TRY(launch_attn_t<_Float16>(a, hd, G, items, st));
     } else {
         const int kind = kv_dtype == DT_I8 ? KV_I8 : kv_dtype == DT_F32 ? KV_F32 : KV_F16;
-        const dim3 grid(split ? a.gx : items, Hkv);
-        const size_t lds = 4 * G * hd * sizeof(float);
+        // chunk grid: one workgroup per chunk of 4 waves, or per sequence (chunk_waves)
+        const dim3 grid(split ? a.gx : nw == 4 ? items : n, Hkv);
+        const size_t lds = (size_t)nw * G * hd * sizeof(float);
         const bool upg = page_size >= 16;  // page ids uniform per wave (page_id)
-#define QH_ATTN_MFMA(K, HDv, KINDv)                                                                    \
-    if (kind == KINDv && hd == HDv) {                                                                  \
-        if (upg) hipLaunchKernelGGL((K<HDv, KINDv, true>), grid, dim3(ACH), lds, st, a, G);            \
-        else hipLaunchKernelGGL((K<HDv, KINDv, false>), grid, dim3(ACH), lds, st, a, G);               \
+#define QH_ATTN_SPLIT(HDv, KINDv)                                                                              \
+    if (kind == KINDv && hd == HDv) {                                                                          \
+        if (upg) hipLaunchKernelGGL((attn_split_kernel<HDv, KINDv, true>), grid, dim3(ACH), lds, st, a, G);    \
+        else hipLaunchKernelGGL((attn_split_kernel<HDv, KINDv, false>), grid, dim3(ACH), lds, st, a, G);       \
     }
+#define QH_ATTN_CHUNK(HDv, KINDv, NWv)                                                                         \
+    if (kind == KINDv && hd == HDv && nw == NWv) {                                                             \
+        if (upg) hipLaunchKernelGGL((attn_mfma_kernel<HDv, KINDv, true, NWv>), grid, dim3(64 * NWv), lds, st, a, G); \
+        else hipLaunchKernelGGL((attn_mfma_kernel<HDv, KINDv, false, NWv>), grid, dim3(64 * NWv), lds, st, a, G);    \
+    }
+#define QH_ATTN_CHUNKS(HDv, KINDv) \
+    QH_ATTN_CHUNK(HDv, KINDv, 4) QH_ATTN_CHUNK(HDv, KINDv, 8) QH_ATTN_CHUNK(HDv, KINDv, 12) QH_ATTN_CHUNK(HDv, KINDv, 16)
         if (split) {
-            QH_ATTN_MFMA(attn_split_kernel, 128, KV_F16) QH_ATTN_MFMA(attn_split_kernel, 64, KV_F16)
-            QH_ATTN_MFMA(attn_split_kernel, 128, KV_I8) QH_ATTN_MFMA(attn_split_kernel, 64, KV_I8)
-            QH_ATTN_MFMA(attn_split_kernel, 128, KV_F32) QH_ATTN_MFMA(attn_split_kernel, 64, KV_F32)
+            QH_ATTN_SPLIT(128, KV_F16) QH_ATTN_SPLIT(64, KV_F16) QH_ATTN_SPLIT(128, KV_I8)
+            QH_ATTN_SPLIT(64, KV_I8) QH_ATTN_SPLIT(128, KV_F32) QH_ATTN_SPLIT(64, KV_F32)
         } else {
-            QH_ATTN_MFMA(attn_mfma_kernel, 128, KV_F16) QH_ATTN_MFMA(attn_mfma_kernel, 64, KV_F16)
-            QH_ATTN_MFMA(attn_mfma_kernel, 128, KV_I8) QH_ATTN_MFMA(attn_mfma_kernel, 64, KV_I8)
-            QH_ATTN_MFMA(attn_mfma_kernel, 128, KV_F32) QH_ATTN_MFMA(attn_mfma_kernel, 64, KV_F32)
+            QH_ATTN_CHUNKS(128, KV_F16) QH_ATTN_CHUNKS(64, KV_F16) QH_ATTN_CHUNKS(128, KV_I8)
+            QH_ATTN_CHUNKS(64, KV_I8) QH_ATTN_CHUNKS(128, KV_F32) QH_ATTN_CHUNKS(64, KV_F32)
         }
-#undef QH_ATTN_MFMA
+#undef QH_ATTN_SPLIT
+#undef QH_ATTN_CHUNK
+#undef QH_ATTN_CHUNKS
         QH_CHECK_HIP(hipGetLastError());
     }
     if (split) {  // a sequence may span several workgroups' shares
@@ -1518,7 +1595,7 @@ int launch_attention(const float* q, const void* kc, const void* vc, uint32_t kv
         if (hd == 128) hipLaunchKernelGGL((attn_merge_kernel<128, true>), mg, dim3(64), 0, st, a);
         else hipLaunchKernelGGL((attn_merge_kernel<64, true>), mg, dim3(64), 0, st, a);
         QH_CHECK_HIP(hipGetLastError());
-    } else if (max_ctx > ACH) {  // some sequence may span several chunks
+    } else if (max_ctx > 64 * nw) {  // some sequence may span several chunks
         const dim3 mg(n, H);
         if (hd == 128) hipLaunchKernelGGL((attn_merge_kernel<128, false>), mg, dim3(64), 0, st, a);
         else if (hd == 64) hipLaunchKernelGGL((attn_merge_kernel<64, false>), mg, dim3(64), 0, st, a);

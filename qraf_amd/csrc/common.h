@@ -199,6 +199,8 @@ size_t attn_workspace_bytes(int n, int H, int Hkv, int hd, int max_ctx);
 // resolves the device address of the no-allocation attention workspace on
 // `device` (current); called once per device by qraf_hip_init
 int attn_scratch_init(int device);
+// raises the dynamic-LDS limit of the wide attention workgroups (qraf_hip_init)
+int attention_init();
 int launch_attention(const float* q, const void* kc, const void* vc, uint32_t kv_dtype, const int32_t* page_table,
                      int max_pages, const int32_t* ctx, int n, int H, int Hkv, int hd, int page_size, float scale,
                      int max_ctx, float* out, void* ws, size_t ws_bytes, hipStream_t st, uint16_t* out_hi = nullptr,
