@@ -50,6 +50,8 @@
 // every operand in fp32 as it is.  attn_decode_kernel (the other shapes, and
 // f32 / fp16 pages on request) is plain fp32 VALU code on the chunk grid:
 // scores with thread = position, output with thread = (head, dimension).
+// attn_few_kernel takes f32 pages where one workgroup per query head (or KV
+// head) does not fill the chip: fp32 VALU code, latency-bound.
 #include <math.h>
 
 #include <algorithm>
@@ -304,6 +306,197 @@ __global__ __launch_bounds__(ACH) void attn_decode_kernel(AttnArgs a) {
         a.part_ml[((size_t)item * a.H + kvh * G + tid) * 2 + 0] = m[tid];
         a.part_ml[((size_t)item * a.H + kvh * G + tid) * 2 + 1] = l[tid];
     }
+}
+
+// ---------------------------------------------------------------------------
+// Few sequences on f32 pages, up to TPW * 256 positions (decode of one or a
+// handful of sequences).  One workgroup per (sequence, G query heads of one KV
+// head) is latency-bound, not rate-bound: the chain is page ids -> K ->
+// scores -> softmax -> V -> sums, and what counts is how many of its links
+// wait for memory, how many barriers it has and how much each SIMD issues.
+// 16 waves; wave w takes the 16-position tiles w, w + 16, ... (TPW of them)
+// whole: the K and V loads of the workgroup are requested together behind the
+// page ids, each wave keeps its own maximum and sum, and the one barrier is in
+// front of the final combination.  SmolLM2-135M shapes, one sequence of up to
+// 256 positions: 7.7 us (VALU kernel) and 7.1 (matrix cores) -> 4.4; 16 of
+// them 8.5 -> 4.7; Qwen2.5-3B shapes (head_dim 128), one: 13.3 -> 6.3.
+//
+// Scores: lanes 4i .. 4i+3 hold position i of the tile, lane quarter j the
+// float4s j, j + 4, j + 8, j + 12 of the row (64 contiguous bytes per load).
+// P.V: lane 16r + c holds dimensions 4c .. 4c+3 of positions 4r .. 4r+3 (a
+// load reads 4 whole rows), whose probabilities lie in the lane's own row of
+// 16.  Every exchange is DPP or a lane-row swap: with 16 waves on one CU the
+// LDS shuffles took longer than the loads (4 heads, 256 positions, one sequence: 7.9 us with
+// LDS shuffles, 6.7 with these, 4.2 with a workgroup per head).
+// Positions past the context read the tile's first row and count as 0.
+// ---------------------------------------------------------------------------
+// lane exchanges without LDS: DPP controls inside rows of 16 lanes (quad_perm
+// for xor 1 and 2, row_ror, row_newbcast), lane-row swaps across them
+template <int CTRL>
+__device__ __forceinline__ int dpp(int x) {
+    return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xF, 0xF, true);
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp(float x) {
+    return __builtin_bit_cast(float, dpp<CTRL>(__builtin_bit_cast(int, x)));
+}
+enum : int { DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E, DPP_ROR4 = 0x124, DPP_ROR8 = 0x128, DPP_BCAST = 0x150 };
+// op of each of four values over the 4 rows of 16 lanes, lane by lane: row r
+// gets value r's (each swap pairs two values, so three swaps serve all four)
+template <typename F>
+__device__ __forceinline__ float over_rows(float x, float y, float z, float w, F op) {
+    auto f = [](unsigned u) { return __builtin_bit_cast(float, u); };
+    auto u = [](float v) { return __builtin_bit_cast(unsigned, v); };
+    const auto a = __builtin_amdgcn_permlane16_swap(u(x), u(y), false, false);
+    const auto b = __builtin_amdgcn_permlane16_swap(u(z), u(w), false, false);
+    const float p = op(f(a[0]), f(a[1])), q = op(f(b[0]), f(b[1]));
+    const auto c = __builtin_amdgcn_permlane32_swap(u(p), u(q), false, false);
+    return op(f(c[0]), f(c[1]));
+}
+template <int HD, int G, int TPW>
+__global__ __launch_bounds__(1024, 4) void attn_few_kernel(AttnArgs a) {
+    constexpr int NW = 16, KQ = HD / 16, VQ = HD / 64;  // float4s of a lane's K quarter, of its V dimensions
+    __shared__ __align__(16) float s_o[NW][G][HD];
+    __shared__ float s_m[NW][G], s_l[NW][G];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int s = blockIdx.x, head = blockIdx.y * G;  // G query heads from this one
+    const int kvh = head / (a.H / a.Hkv);
+    const int i = lane >> 2, j = lane & 3, r = lane >> 4, c = lane & 15;
+
+    // requested together: the context length, the page id of the lane's
+    // position per tile (table index clamped into the table), q
+    const int ctx_raw = a.ctx[s];
+    int pg[TPW];
+#pragma unroll
+    for (int t = 0; t < TPW; t++)
+        pg[t] = a.page_table[(size_t)s * a.max_pages + min(16 * (wave + NW * t) + i, a.max_ctx - 1) / a.page_size];
+    const float* qp = a.q + ((size_t)s * a.H + head) * HD + 4 * j;
+    float4 q[G][KQ];
+#pragma unroll
+    for (int h = 0; h < G; h++)
+#pragma unroll
+        for (int k = 0; k < KQ; k++) q[h][k] = *(const float4*)(qp + h * HD + 16 * k);
+    const int ctx = min(ctx_raw, a.max_ctx);
+    if (ctx <= 0) return;
+
+    const float* kc = (const float*)a.kc;
+    const float* vc = (const float*)a.vc;
+    float4 kr[TPW][KQ], vr[TPW][4][VQ];
+#pragma unroll
+    for (int t = 0; t < TPW; t++) {
+        const int p0 = 16 * (wave + NW * t);
+        if (p0 < ctx) {  // wave-uniform
+            // row of position p0 + x on page id; past the context p0's row
+            const int first = __builtin_amdgcn_readfirstlane(pg[t]);
+            auto row = [&](int x, int id) {
+                const bool in = p0 + x < ctx;
+                return (((size_t)(in ? id : first) * a.Hkv + kvh) * a.page_size + (in ? p0 + x : p0) % a.page_size) * HD;
+            };
+            const float* kp = kc + row(i, pg[t]) + 4 * j;
+#pragma unroll
+            for (int k = 0; k < KQ; k++) kr[t][k] = *(const float4*)(kp + 16 * k);
+            auto vrow = [&](int x, int id, float4 (&v)[VQ]) {
+                const float* vp = vc + row(x, id) + 4 * c;
+#pragma unroll
+                for (int y = 0; y < VQ; y++) v[y] = *(const float4*)(vp + 64 * y);
+            };
+            vrow(4 * r + 0, dpp<DPP_BCAST + 0>(pg[t]), vr[t][0]);
+            vrow(4 * r + 1, dpp<DPP_BCAST + 4>(pg[t]), vr[t][1]);
+            vrow(4 * r + 2, dpp<DPP_BCAST + 8>(pg[t]), vr[t][2]);
+            vrow(4 * r + 3, dpp<DPP_BCAST + 12>(pg[t]), vr[t][3]);
+        }
+    }
+
+    float sc[TPW][G], m[G], l[G];
+    float4 o[G][VQ];
+#pragma unroll
+    for (int h = 0; h < G; h++) {
+        m[h] = -INFINITY;
+        l[h] = 0.f;
+#pragma unroll
+        for (int y = 0; y < VQ; y++) o[h][y] = float4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int t = 0; t < TPW; t++) {
+        const int p0 = 16 * (wave + NW * t);
+        if (p0 < ctx) {
+#pragma unroll
+            for (int h = 0; h < G; h++) {
+                float x = 0.f;
+#pragma unroll
+                for (int k = 0; k < KQ; k++) {
+                    x = __builtin_fmaf(q[h][k].x, kr[t][k].x, x);
+                    x = __builtin_fmaf(q[h][k].y, kr[t][k].y, x);
+                    x = __builtin_fmaf(q[h][k].z, kr[t][k].z, x);
+                    x = __builtin_fmaf(q[h][k].w, kr[t][k].w, x);
+                }
+                x += dpp<DPP_XOR1>(x);
+                x += dpp<DPP_XOR2>(x);
+                x *= a.scale;  // attention.cpp:134: dot * scale
+                sc[t][h] = p0 + i < ctx ? x : -INFINITY;
+                m[h] = fmaxf(m[h], sc[t][h]);
+            }
+        }
+    }
+    float mx = over_rows(m[0], m[G > 1 ? 1 : 0], m[G > 2 ? 2 : 0], m[G > 3 ? 3 : 0], [](float x, float y) { return fmaxf(x, y); });
+    mx = fmaxf(mx, dpp<DPP_ROR4>(mx));
+    mx = fmaxf(mx, dpp<DPP_ROR8>(mx));  // row h: head h's maximum
+#pragma unroll
+    for (int h = 0; h < G; h++)
+        m[h] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mx), 16 * h));
+#pragma unroll
+    for (int t = 0; t < TPW; t++) {
+        const int p0 = 16 * (wave + NW * t);
+        if (p0 < ctx) {
+#pragma unroll
+            for (int h = 0; h < G; h++) {
+                const float p = p0 + i < ctx ? __expf(sc[t][h] - m[h]) : 0.f;
+                l[h] += p;
+                auto add = [&](float w, const float4 (&v)[VQ]) {
+#pragma unroll
+                    for (int y = 0; y < VQ; y++) {
+                        o[h][y].x = __builtin_fmaf(w, v[y].x, o[h][y].x);
+                        o[h][y].y = __builtin_fmaf(w, v[y].y, o[h][y].y);
+                        o[h][y].z = __builtin_fmaf(w, v[y].z, o[h][y].z);
+                        o[h][y].w = __builtin_fmaf(w, v[y].w, o[h][y].w);
+                    }
+                };
+                add(dpp<DPP_BCAST + 0>(p), vr[t][0]);
+                add(dpp<DPP_BCAST + 4>(p), vr[t][1]);
+                add(dpp<DPP_BCAST + 8>(p), vr[t][2]);
+                add(dpp<DPP_BCAST + 12>(p), vr[t][3]);
+            }
+        }
+    }
+    if (16 * wave < ctx) {  // the wave holds positions
+        auto sum = [](float x, float y) { return x + y; };
+        float ls = over_rows(l[0], l[G > 1 ? 1 : 0], l[G > 2 ? 2 : 0], l[G > 3 ? 3 : 0], sum);
+        ls += dpp<DPP_ROR4>(ls);
+        ls += dpp<DPP_ROR8>(ls);
+        if (c == 0 && r < G) {
+            s_m[wave][r] = mx;
+            s_l[wave][r] = ls;
+        }
+#pragma unroll
+        for (int h = 0; h < G; h++)
+#pragma unroll
+            for (int y = 0; y < VQ; y++)
+                s_o[wave][h][64 * y + 4 * c + r] = over_rows(o[h][y].x, o[h][y].y, o[h][y].z, o[h][y].w, sum);
+    }
+    __syncthreads();
+    if (tid >= G * HD) return;
+    const int h = tid / HD, d = tid % HD;
+    const int nw = min(NW, (ctx + 15) >> 4);  // waves with positions
+    float M = s_m[0][h];
+    for (int v = 1; v < nw; v++) M = fmaxf(M, s_m[v][h]);
+    float O = 0.f, L = 0.f;
+    for (int v = 0; v < nw; v++) {
+        const float e = __expf(s_m[v][h] - M);
+        O = __builtin_fmaf(s_o[v][h][d], e, O);
+        L = __builtin_fmaf(s_l[v][h], e, L);
+    }
+    attn_store(a, ((size_t)s * a.H + head) * HD + tid, O / L);
 }
 
 // ---------------------------------------------------------------------------
@@ -1460,6 +1653,26 @@ size_t attn_workspace_bytes(int n, int H, int Hkv, int hd, int max_ctx) {
 // 3: the plain fp32 VALU kernel for f32 and fp16 pages (int8 pages: automatic)
 static int g_attn_form = 0;
 
+// Query heads per workgroup of attn_few_kernel, 0 for another kernel.  A
+// workgroup per query head while every one has a CU of its own: the heads of
+// a group read the same K and V again, from caches, but each SIMD issues one
+// head's work (one KV head x 4 heads, ctx 128-256, 64 sequences: 7.6 us with 4
+// heads a workgroup, 4.8 with one; 85 sequences, past the 256 CUs, take 4
+// heads: 6.7, the matrix cores 8.6).  TPW 1, 2, 4 tiles per wave hold 256, 512
+// and (head_dim 64) 1,024 positions; measured against the matrix-core kernels
+// at 1-28 sequences: up to 256 positions 1.5-3.0 times as fast, 512 1.1-2.2
+// times, 1,024 1.1-1.5 times.  Two to four heads a workgroup beyond 256 of
+// them: 3 heads x 85 sequences of 256 positions 11.4 -> 8.9 us, of 512 18.4 ->
+// 13.3; 4 heads at 512 positions spill (14.6 -> 16.5 us) and stay out.
+static int few_heads(int n, int H, int Hkv, int hd, int max_ctx) {
+    const int G = H / Hkv;
+    if (n * H <= 256 && max_ctx <= (hd == 64 ? 1024 : 512)) return 1;
+    return hd == 64 && max_ctx <= 512 && n * Hkv <= 256 && (G < 4 || (G == 4 && max_ctx <= 256)) ? G : 0;
+}
+
+// query heads per KV head that attn_decode_kernel is built for at head_dim 64
+static bool valu_group(int G) { return G <= 4 || G == 6 || G == 8 || G == 12 || G == 16; }
+
 // Waves per workgroup of the matrix-core chunk grid, one 64-position tile
 // each.  Contexts that may pass one 256-position chunk get a workgroup of 8,
 // 12 or 16 waves where that holds the whole context: no partials and no merge
@@ -1548,13 +1761,28 @@ int launch_attention(const float* q, const void* kc, const void* vc, uint32_t kv
     a.scale = scale;
     const int G = H / Hkv;
     const bool mfma_shape = (hd == 64 || hd == 128) && G <= 16 && page_size % 4 == 0 && ps_pow2;
-    // One sequence of at most one 256-position chunk on f32 pages at
-    // head_dim 64 (batch-1 decode of a small model): the VALU kernel, whose
-    // one round of K/V loads beats the matrix-core kernel's pipelined tiles
-    // when a single workgroup per KV head is all there is (SmolLM2-135M
-    // architecture decode on MI355X: 1,373 against 1,296 tok/s)
-    const bool single_f32 = kv_dtype == DT_F32 && hd == 64 && n == 1 && max_ctx <= ACH && g_attn_form == 0;
-    const bool valu = !mfma_shape || (g_attn_form == 3 && kv_dtype != DT_I8) || single_f32;
+    // one sequence of one 256-position chunk on f32 pages at head_dim 64 whose
+    // group the VALU kernel was not built for stays that kernel's to refuse
+    const bool refused = kv_dtype == DT_F32 && hd == 64 && n == 1 && max_ctx <= ACH && !valu_group(G) && g_attn_form == 0;
+    const int few = kv_dtype == DT_F32 && mfma_shape && g_attn_form == 0 && !refused
+                        ? few_heads(n, H, Hkv, hd, max_ctx) : 0;
+    if (few) {
+        const dim3 grid(n, H / few);
+        const int tpw = (max_ctx + 255) / 256;  // 16-position tiles per wave
+        if (hd == 128 && tpw == 1) hipLaunchKernelGGL((attn_few_kernel<128, 1, 1>), grid, dim3(1024), 0, st, a);
+        else if (hd == 128) hipLaunchKernelGGL((attn_few_kernel<128, 1, 2>), grid, dim3(1024), 0, st, a);
+        else if (tpw > 2) hipLaunchKernelGGL((attn_few_kernel<64, 1, 4>), grid, dim3(1024), 0, st, a);
+#define QH_ATTN_FEW(Gv)                                                                                      \
+    else if (few == Gv) {                                                                                    \
+        if (tpw == 1) hipLaunchKernelGGL((attn_few_kernel<64, Gv, 1>), grid, dim3(1024), 0, st, a);    \
+        else hipLaunchKernelGGL((attn_few_kernel<64, Gv, 2>), grid, dim3(1024), 0, st, a);                   \
+    }
+        QH_ATTN_FEW(1) QH_ATTN_FEW(2) QH_ATTN_FEW(3) QH_ATTN_FEW(4)
+#undef QH_ATTN_FEW
+        QH_CHECK_HIP(hipGetLastError());
+        return QRAF_HIP_OK;
+    }
+    const bool valu = !mfma_shape || (g_attn_form == 3 && kv_dtype != DT_I8) || refused;
     const bool split = !valu && (g_attn_form == 2 || (g_attn_form != 1 && items > 1024));
     const int nw = valu || split ? 4 : chunk_waves(n, Hkv, max_ctx);
     if (valu) {  // the plain fp32 VALU kernel

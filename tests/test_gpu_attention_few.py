@@ -1,0 +1,47 @@
+"""Decode attention of few sequences on f32 pages (16 waves, one 16-position
+tile each and up to four in turn) against the oracle: context lengths around
+the edges of a tile, of the 16 waves and of each number of tiles per wave,
+every number of heads a workgroup takes, the workgroup counts on both sides of
+the choice, page sizes of 4 to 64, NaN behind each context.  The tolerance is
+that of the other forms: only the order of the fp32 sums differs."""
+import numpy as np
+import pytest
+
+from oracle import pyoracle as po
+from tests.test_gpu_attention import build_cache, check, oracle_attention, run_attention
+
+pytestmark = pytest.mark.gpu
+
+EDGES = [1, 2, 15, 16, 17, 31, 33, 63, 255, 256, 257, 272, 273, 511, 512, 513, 768, 769, 1009, 1024, 1025]
+
+
+def run(hip, n, H, Hkv, hd, ps, ctxs):
+    rng = np.random.default_rng(n * H + hd + max(ctxs))
+    table, K, V, _ = build_cache(rng, ctxs, Hkv, hd, ps, po.F32, poison=True)
+    q = (rng.standard_normal((n, H * hd)) * 2).astype(np.float32)
+    got = run_attention(hip, q, table, K, V, ctxs, H, Hkv, hd, ps, po.F32, max(ctxs), repeats=2)
+    assert np.array_equal(got[0], got[1])
+    check(got[0], oracle_attention(q, table, K, V, ctxs, H, Hkv, hd, ps))
+
+
+@pytest.mark.parametrize("H,Hkv,hd", [(9, 3, 64), (10, 2, 64), (16, 1, 64), (16, 2, 128), (8, 8, 128)])
+@pytest.mark.parametrize("ps", [4, 16, 64])
+def test_one_sequence(hip, H, Hkv, hd, ps):
+    for c in EDGES:
+        if (H // Hkv, hd) == (5, 64) and c <= 256:
+            continue  # one sequence of this group: refused
+        run(hip, 1, H, Hkv, hd, ps, [c])
+
+
+@pytest.mark.parametrize("H,Hkv,hd", [(3, 3, 64), (6, 3, 64), (9, 3, 64), (12, 3, 64), (15, 3, 64), (16, 2, 128)])
+@pytest.mark.parametrize("n", [15, 29, 43, 85, 86])
+@pytest.mark.parametrize("most", [48, 256, 512, 513, 1024])
+def test_ragged_batches(hip, H, Hkv, hd, n, most):
+    edges = [c for c in EDGES if c <= most][::-1][:n]
+    rng = np.random.default_rng(n + most)
+    run(hip, n, H, Hkv, hd, 16, edges + rng.integers(1, most + 1, n - len(edges)).tolist())
+
+
+def test_group_without_a_kernel_stays_refused(hip):
+    with pytest.raises(RuntimeError, match="group 5"):
+        run(hip, 1, 10, 2, 64, 16, [40])
