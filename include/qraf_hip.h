@@ -193,7 +193,9 @@ uint64_t qraf_hip_attention_workspace_bytes(int32_t n_seqs, int32_t n_heads, int
  * 1 = one workgroup per (sequence, 256-position chunk), 2 = balanced split
  * of the batch's 64-position tiles over the resident workgroups,
  * 0 = automatic (default: the split when n_seqs * ceil(max_ctx / 256)
- * exceeds 1024, else the chunk grid), 3 = the plain fp32 VALU kernel for F32
+ * exceeds 1024; else the chunk grid, whose workgroups hold a whole context
+ * of up to 1,024 positions where that is the faster form, or on F32 pages the
+ * small-batch kernel), 3 = the plain fp32 VALU kernel for F32
  * and F16 pages (I8 pages: automatic).  Results agree within the attention
  * tolerance, not bit for bit. */
 int qraf_hip_set_attention_tuning(int32_t form);
@@ -249,8 +251,8 @@ int qraf_hip_split_bf16_dev(const float* x, uint16_t* x_hi, uint16_t* x_lo, int3
  * workgroup (128 or 256 weight rows), splits > 0 forces the split count,
  * pipe 1 / -1 forces the pipelined tiled kernel on / off, batch_chunk 16,
  * 32, 64 or 128 caps the batch rows one workgroup covers; 0 restores the
- * automatic choice.  Affects the workspace queries too.  No counterpart in
- * the reference (a performance knob). */
+ * automatic choice, which alone takes the 32x32 form.  Affects the workspace
+ * queries too.  No counterpart in the reference (a performance knob). */
 int qraf_hip_set_qgemm_tuning(int waves, int splits, int pipe, int batch_chunk);
 /* Work schedule of the pipelined GEMM (batches over 32 rows, tile-major
  * weights): mode 1 = stream-K (each resident workgroup takes an equal share
@@ -267,7 +269,8 @@ int qraf_hip_set_qgemm_schedule(int32_t mode, int32_t min_blocks);
 /* Wave-split form of the tile-major GEMM (each workgroup's 4 waves take its
  * quant blocks in turn and meet once in LDS at the end): mode 1 selects it
  * for every tiled batch over 16 rows, -1 never, 0 (the default) for batches
- * of 17-32 rows and of 33-64 rows below 16384 output rows, unless
+ * of 17-32 rows where the 32x32 form (the automatic choice of most batches
+ * over 16 rows while no form or split count is forced) does not run, unless
  * qraf_hip_set_qgemm_tuning forces another form;
  * tiles_per_workgroup 2, 3 or 4 fixes its 16-row weight tiles per workgroup
  * (0: automatic).  Affects the workspace queries and the SwiGLU-epilogue

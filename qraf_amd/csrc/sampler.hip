@@ -493,8 +493,8 @@ __global__ __launch_bounds__(SNT) void sample_rows_kernel(const float* __restric
     // ---- one read of the row and a search among sub-range maxima (see the file
     // comment).  Bound by the row's bytes (one workgroup per row; the search passes
     // below read the row once each): MI355X, 128 rows x 151936, top-k 40, top-p 0.9:
-    // 114 -> 28 us (77.8 MB read once: 15 us at the rate of a large copy).  Left to the searches below: maxima that are not finite
-    // (masked rows) and more than CAND_CAP values at the bound.
+    // 114 -> 28 us (77.8 MB read once: 15 us at the rate of a large copy).  Left
+    // to the searches below: maxima that are not finite (masked rows) and more than CAND_CAP values at the bound.
     if (!fast && !big && (V & 3) == 0 && V >= SUB_MIN && cutoff <= SUB_CUT) {
         const float4* l4 = (const float4*)l;
         const int V4 = V >> 2, Q = (V4 + NSUB - 1) / NSUB;  // float4s per sub-range
