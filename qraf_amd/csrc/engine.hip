@@ -677,7 +677,7 @@ int qraf_engine_create(const qraf_model_config* cfg, const qraf_engine_options* 
     }
     if (e->part_ws_bytes) A(e->part_ws, e->part_ws_bytes);
 #undef A
-    if (hipMemset(e->attn_ws, 0, e->attn_ws_bytes) != hipSuccess)
+    if (hipMemsetAsync(e->attn_ws, 0, e->attn_ws_bytes, e->stream) != hipSuccess)
         return fail(set_error(QRAF_HIP_ERR_HIP, "engine: workspace set-up failed"));
     for (int k = 0; k < 2; k++)
         if (hipHostMalloc((void**)&e->h_in[k], e->in_words * 4, hipHostMallocDefault) != hipSuccess ||
@@ -688,7 +688,8 @@ int qraf_engine_create(const qraf_model_config* cfg, const qraf_engine_options* 
     {
         std::vector<float> tab((size_t)e->capacity * hd);
         qraf_hip_rope_table_host(e->capacity, hd, c.rope_theta, tab.data());
-        if (hipMemcpy(e->rope, tab.data(), tab.size() * 4, hipMemcpyHostToDevice) != hipSuccess)
+        if (hipMemcpyAsync(e->rope, tab.data(), tab.size() * 4, hipMemcpyHostToDevice, e->stream) != hipSuccess ||
+            hipStreamSynchronize(e->stream) != hipSuccess)
             return fail(set_error(QRAF_HIP_ERR_HIP, "engine: rope table upload failed"));
     }
     {
@@ -749,7 +750,10 @@ int qraf_engine_set_tensor(qraf_engine* e, const char* name, uint32_t dtype, uin
         return QRAF_HIP_OK;
     };
     auto upload = [&](void* dst, const void* src, size_t n) -> int {
-        QH_CHECK_HIP(hipMemcpy(dst, src, n, hipMemcpyHostToDevice));
+        // on the engine's stream: a copy on the legacy stream fails, and breaks
+        // the capture, while another thread's engine captures a step
+        QH_CHECK_HIP(hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, e->stream));
+        QH_CHECK_HIP(hipStreamSynchronize(e->stream));
         return QRAF_HIP_OK;
     };
     auto ensure = [&](uint8_t** p, size_t n) -> int {
@@ -807,7 +811,7 @@ int qraf_engine_set_tensor(qraf_engine* e, const char* name, uint32_t dtype, uin
             QH_REQUIRE(rows == t.r && bytes >= (uint64_t)t.r * 4, QRAF_HIP_ERR_INVALID, "set_tensor %s: bad shape", name);
             if (!L.bqkv) {
                 QH_TRY(ensure((uint8_t**)&L.bqkv, (size_t)e->qkvd * 4));
-                QH_CHECK_HIP(hipMemset(L.bqkv, 0, (size_t)e->qkvd * 4));
+                QH_CHECK_HIP(hipMemsetAsync(L.bqkv, 0, (size_t)e->qkvd * 4, e->stream));
             }
             L.has_bias = true;
             return upload(L.bqkv + t.off, data, (size_t)t.r * 4);
@@ -852,7 +856,9 @@ int qraf_engine_set_tensor(qraf_engine* e, const char* name, uint32_t dtype, uin
         QH_TRY(ensure(&L.wgu, 2 * n));
         gdt = dtype;
         L.have |= t.bit;
-        QH_CHECK_HIP(hipMemcpy2D(L.wgu + (size_t)t.off * rb, 2 * rb, data, rb, rb, t.r, hipMemcpyHostToDevice));
+        QH_CHECK_HIP(hipMemcpy2DAsync(L.wgu + (size_t)t.off * rb, 2 * rb, data, rb, rb, t.r, hipMemcpyHostToDevice,
+                                      e->stream));
+        QH_CHECK_HIP(hipStreamSynchronize(e->stream));
         return QRAF_HIP_OK;
     }
     return QRAF_HIP_OK;  // unknown per-layer tensor: not read by the LLaMA path
