@@ -328,7 +328,8 @@ __global__ __launch_bounds__(ACH) void attn_decode_kernel(AttnArgs a) {
 // 16.  Every exchange is DPP or a lane-row swap: with 16 waves on one CU the
 // LDS shuffles took longer than the loads (4 heads, 256 positions, one sequence: 7.9 us with
 // LDS shuffles, 6.7 with these, 4.2 with a workgroup per head).
-// Positions past the context read the tile's first row and count as 0.
+// Positions past the context read the tile's first row and count as 0, as do
+// scores of -inf: a wave may hold nothing else.
 // ---------------------------------------------------------------------------
 // lane exchanges without LDS: DPP controls inside rows of 16 lanes (quad_perm
 // for xor 1 and 2, row_ror, row_newbcast), lane-row swaps across them
@@ -451,7 +452,7 @@ __global__ __launch_bounds__(1024, 4) void attn_few_kernel(AttnArgs a) {
         if (p0 < ctx) {
 #pragma unroll
             for (int h = 0; h < G; h++) {
-                const float p = p0 + i < ctx ? __expf(sc[t][h] - m[h]) : 0.f;
+                const float p = sc[t][h] == -INFINITY ? 0.f : __expf(sc[t][h] - m[h]);  // m may be -inf
                 l[h] += p;
                 auto add = [&](float w, const float4 (&v)[VQ]) {
 #pragma unroll
@@ -492,7 +493,7 @@ __global__ __launch_bounds__(1024, 4) void attn_few_kernel(AttnArgs a) {
     for (int v = 1; v < nw; v++) M = fmaxf(M, s_m[v][h]);
     float O = 0.f, L = 0.f;
     for (int v = 0; v < nw; v++) {
-        const float e = __expf(s_m[v][h] - M);
+        const float e = s_m[v][h] == -INFINITY ? 0.f : __expf(s_m[v][h] - M);
         O = __builtin_fmaf(s_o[v][h][d], e, O);
         L = __builtin_fmaf(s_l[v][h], e, L);
     }

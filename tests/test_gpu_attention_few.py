@@ -45,3 +45,29 @@ def test_ragged_batches(hip, H, Hkv, hd, n, most):
 def test_group_without_a_kernel_stays_refused(hip):
     with pytest.raises(RuntimeError, match="group 5"):
         run(hip, 1, 10, 2, 64, 16, [40])
+
+
+@pytest.mark.parametrize("how", ["overflow", "infinite"])
+@pytest.mark.parametrize("n,H,Hkv,hd,ctx", [
+    # n * H <= 256: a workgroup per query head; beyond it (head_dim 64) one per KV head; the matrix cores
+    (1, 9, 3, 64, 17), (1, 9, 3, 64, 250), (28, 9, 3, 64, 257), (29, 9, 3, 64, 257), (64, 4, 1, 64, 49),
+    (65, 4, 1, 64, 49), (16, 9, 3, 64, 700), (1, 16, 2, 128, 33), (16, 16, 2, 128, 500), (17, 16, 2, 128, 500),
+    (86, 9, 3, 64, 200)])
+def test_scores_of_minus_infinity(hip, n, H, Hkv, hd, ctx, how):
+    """Keys whose score is -inf count as nothing (exp(-inf - max) = 0 in the
+    oracle's softmax): the only position of the last tile, a whole tile, and
+    single positions, through products that overflow and through an infinite
+    key element."""
+    ps = 16
+    ctxs = [ctx - 16 * (s % 2) if ctx > 32 else ctx for s in range(n)]  # ctx % 16 is the same for all
+    rng = np.random.default_rng(n + ctx + hd)
+    table, K, V, _ = build_cache(rng, ctxs, Hkv, hd, ps, po.F32, poison=True)
+    q = (rng.standard_normal((n, H * hd)) * 2).astype(np.float32)
+    q.reshape(n, H, hd)[:, :, 5] = 2 + np.abs(q.reshape(n, H, hd)[:, :, 5])
+    low = np.float32(-np.inf if how == "infinite" else -3e38)  # times q > 2: past the range of fp32
+    for s, c in enumerate(ctxs):
+        last = c - 1 if c % 16 == 1 else c - 3
+        for t in [last, 3] + (list(range(16, 32)) if c > 32 else []):
+            K[table[s, t // ps], :, t % ps, 5] = low
+    got = run_attention(hip, q, table, K, V, ctxs, H, Hkv, hd, ps, po.F32, max(ctxs))
+    check(got[0], oracle_attention(q, table, K, V, ctxs, H, Hkv, hd, ps))
