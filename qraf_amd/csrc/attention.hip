@@ -450,6 +450,12 @@ __global__ __launch_bounds__(1024, 4) void attn_few_kernel(AttnArgs a) {
     for (int t = 0; t < TPW; t++) {
         const int p0 = 16 * (wave + NW * t);
         if (p0 < ctx) {
+            if (p0 + 16 > ctx)  // the first row's repetitions: 0 times an infinity would be NaN
+#pragma unroll
+                for (int x = 0; x < 4; x++)
+#pragma unroll
+                    for (int y = 0; y < VQ; y++)
+                        if (p0 + 4 * r + x >= ctx) vr[t][x][y] = float4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int h = 0; h < G; h++) {
                 const float p = sc[t][h] == -INFINITY ? 0.f : __expf(sc[t][h] - m[h]);  // m may be -inf

@@ -71,3 +71,23 @@ def test_scores_of_minus_infinity(hip, n, H, Hkv, hd, ctx, how):
             K[table[s, t // ps], :, t % ps, 5] = low
     got = run_attention(hip, q, table, K, V, ctxs, H, Hkv, hd, ps, po.F32, max(ctxs))
     check(got[0], oracle_attention(q, table, K, V, ctxs, H, Hkv, hd, ps))
+
+
+@pytest.mark.parametrize("n,H,Hkv,hd,ctx", [(1, 9, 3, 64, 17), (1, 9, 3, 64, 62), (28, 9, 3, 64, 250), (40, 8, 4, 64, 41),
+                                            (16, 9, 3, 64, 600), (1, 16, 2, 128, 33), (16, 16, 2, 128, 300)])
+def test_infinite_values_stay_infinite(hip, n, H, Hkv, hd, ctx):
+    """An infinite element of V makes its output element infinite, as in the
+    oracle, also at the position whose row the lanes past the context read."""
+    ps = 16
+    rng = np.random.default_rng(n + ctx)
+    table, K, V, _ = build_cache(rng, [ctx] * n, Hkv, hd, ps, po.F32, poison=True)
+    q = rng.standard_normal((n, H * hd)).astype(np.float32)
+    first = (ctx - 1) // 16 * 16  # of the last tile
+    for s in range(n):
+        V[table[s, first // ps], :, first % ps, 7] = np.inf
+        V[table[s, 0], :, 1, 9] = -np.inf
+    got = run_attention(hip, q, table, K, V, [ctx] * n, H, Hkv, hd, ps, po.F32, ctx)[0]
+    want = oracle_attention(q, table, K, V, [ctx] * n, H, Hkv, hd, ps)
+    inf = np.isinf(want)
+    assert inf.sum() == 2 * n * H and np.array_equal(got[inf], want[inf])
+    check(got[~inf], want[~inf])
