@@ -1742,17 +1742,12 @@ int set_qgemm_tuning(int waves, int splits, int pipe, int mchunk) {
 
 size_t qgemm_workspace_bytes(uint32_t dtype, int N, int K, int M, bool tiled) {
     if ((dtype != DT_Q8_0 && dtype != DT_Q4_0) || N <= 0 || K <= 0 || K % 32 || M <= 0) return 0;
-    // covers the plan with and without the 32x32 kernel: one allocation serves the
-    // product whichever form a later tuning call selects
-    const size_t rb = q_row_bytes(dtype, 32, K);
-    return std::max(qgemm_plan(dtype, N, K, M, rb, tiled).ws_bytes, qgemm_plan(dtype, N, K, M, rb, tiled, false).ws_bytes);
+    return qgemm_plan(dtype, N, K, M, q_row_bytes(dtype, 32, K), tiled).ws_bytes;
 }
 
 size_t qgemm_partials_bytes(uint32_t dtype, int N, int K, int M, bool tiled) {
     if ((dtype != DT_Q8_0 && dtype != DT_Q4_0) || N <= 0 || K <= 0 || K % 32 || M <= 0) return 0;
-    const size_t rb = q_row_bytes(dtype, 32, K);
-    const int S = std::max(qgemm_plan(dtype, N, K, M, rb, tiled).S, qgemm_plan(dtype, N, K, M, rb, tiled, false).S);
-    return (size_t)S * M * N * 4;
+    return (size_t)qgemm_plan(dtype, N, K, M, q_row_bytes(dtype, 32, K), tiled).S * M * N * 4;
 }
 
 int launch_split_bf16(const float* x, uint16_t* hi, uint16_t* lo, int M, int K, int op, float* xout, hipStream_t s,
@@ -1921,21 +1916,23 @@ int launch_qgemm(const void* W, uint32_t dtype, int bs, int N, int K, const uint
     const int nb = K / 32;
     QgPlan p = qgemm_plan(dtype, N, K, M, rb, tiled);
     float* part = nullptr;
+    const bool aligned = ws && (((uintptr_t)ws) & 15) == 0;
+    const auto resplit = [&](int S) {  // at most S splits, of whole units of the plan's kernel
+        const int unit = p.wide ? 2 : (p.kwR || p.kxT) ? 1 : (p.pipe ? 1 : 2) * p.KC;
+        p.bps = ((nb + S - 1) / S + unit - 1) / unit * unit;
+        p.S = (nb + p.bps - 1) / p.bps;
+        p.skG = 0;
+    };
     if (slices) {  // partials mode: S slices [S][M][N] in ws, summed by the caller's next kernel
-        QH_REQUIRE(ws && ws_bytes >= (size_t)p.S * M * N * 4 && (((uintptr_t)ws) & 15) == 0 && !add,
-                   QRAF_HIP_ERR_INVALID, "qgemm: partials need a workspace of %zu bytes and no residual",
-                   (size_t)p.S * M * N * 4);
+        const size_t fit = ws_bytes / ((size_t)M * N * 4);
+        QH_REQUIRE(aligned && fit >= 1 && !add, QRAF_HIP_ERR_INVALID,
+                   "qgemm: partials need a workspace of at least %zu bytes and no residual", (size_t)M * N * 4);
+        if ((size_t)p.S > fit) resplit((int)fit);  // sized under other tuning
         part = (float*)ws;
         *slices = p.S;
     } else if (p.S > 1) {
-        if (ws && ws_bytes >= p.ws_bytes && (((uintptr_t)ws) & 15) == 0) {
-            part = (float*)ws;
-        } else {  // no (or too small a) workspace: one split
-            p.S = 1;
-            p.skG = 0;
-            const int unit = p.wide ? 2 : (p.kwR || p.kxT) ? 1 : (p.pipe ? 1 : 2) * p.KC;
-            p.bps = (nb + unit - 1) / unit * unit;
-        }
+        if (aligned && ws_bytes >= p.ws_bytes) part = (float*)ws;
+        else resplit(1);  // no (or too small a) workspace
     }
     QH_REQUIRE(p.mchunks <= 65535, QRAF_HIP_ERR_INVALID, "qgemm: batch %d too large", M);
     const dim3 grid = p.skG > 0 ? dim3(p.skG, 1, 1) : dim3(p.ntiles, p.S, p.mchunks);

@@ -939,3 +939,31 @@ def test_scheduler_penalties_on_device(hip):
     finally:
         e.close()
         m.close()
+
+
+def test_gemm_tuning_after_creation(hip):
+    """A GEMM tuning that asks for more split-K slices than the engine's
+    partial workspace was sized for runs with fewer: the step succeeds and its
+    logits stay within the bar."""
+    kw, seed = SMALL["q4_gqa8_hd128"]
+    m = oracle_model(kw, seed)
+    prompt = [po.lib().or_gen_token(seed, i, kw["vocab"]) for i in range(70)]
+    m.reset()
+    want = np.stack([m.forward(t, pos) for pos, t in enumerate(prompt)])
+    tf = upload(m, kw, max_batch=128)
+    e, call = tf.engine, hip._lib.call
+    try:
+        for rows in (40, 70):
+            for tuning, sched in (((0, 0, 0, 0), 0), ((0, 64, 0, 0), 0), ((0, 0, 1, 0), 0), ((0, 16, 3, 0), 0),
+                                  ((0, 0, 2, 128), 1)):
+                print(f"engine step of {rows} rows, GEMM tuning {tuning}, schedule {sched}", flush=True)
+                call("qraf_hip_set_qgemm_tuning", *tuning)
+                call("qraf_hip_set_qgemm_schedule", sched, 1 if sched else 0)
+                sid = e.seq_create()
+                lg, _ = e.step([sid] * rows, prompt[:rows], list(range(rows)), logits=True)
+                e.seq_release(sid)
+                check_logits(lg, want[:rows], f"{rows} rows, {tuning}")
+    finally:
+        call("qraf_hip_set_qgemm_tuning", 0, 0, 0, 0)
+        call("qraf_hip_set_qgemm_schedule", 0, 0)
+        e.close()
