@@ -249,10 +249,13 @@ int qraf_hip_split_bf16_dev(const float* x, uint16_t* x_hi, uint16_t* x_lo, int3
                             void* stream);
 /* Tuning of the batched GEMM for batches over 32 rows: waves 4 or 8 per
  * workgroup (128 or 256 weight rows), splits > 0 forces the split count,
- * pipe 1 / -1 forces the pipelined tiled kernel on / off, batch_chunk 16,
- * 32, 64 or 128 caps the batch rows one workgroup covers; 0 restores the
- * automatic choice, which alone takes the 32x32 form.  Affects the workspace
- * queries too.  No counterpart in the reference (a performance knob). */
+ * pipe 1 / -1 forces the pipelined tiled kernel on / off, 2 its narrow form,
+ * 3 the row-split kernel (batches over 16 rows), 4..7 the 32x32 kernel's
+ * tiles of 128 x 128, 64 x 128, 64 x 64 and 32 x 64 batch x weight rows
+ * (batches over 16 rows), batch_chunk 16, 32, 64 or 128 caps the batch rows
+ * one workgroup covers; 0 restores the automatic choice.  Affects the
+ * workspace queries too.  No counterpart in the reference (a performance
+ * knob). */
 int qraf_hip_set_qgemm_tuning(int waves, int splits, int pipe, int batch_chunk);
 /* Work schedule of the pipelined GEMM (batches over 32 rows, tile-major
  * weights): mode 1 = stream-K (each resident workgroup takes an equal share

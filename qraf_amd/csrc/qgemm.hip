@@ -1376,12 +1376,15 @@ struct QgPlan {
 static int g_qg_waves = 0;   // 4 or 8 waves per workgroup for batch tiles > 32 rows
 static int g_qg_splits = 0;  // forced split count
 static int g_qg_pipe = 0;    // 1: pipelined kernel for every tiled batch over 32 rows, 2: its narrow
-                             // 4-wave form, -1: never
+                             // 4-wave form, -1: never, 3: row-split kernel over 16 rows, 4 + f: form f
+                             // of the 32x32 kernel over 16 rows
 static int g_qg_mchunk = 0;  // batch rows per workgroup at most (0: QG_MCHUNK)
 static int g_qg_sched = 0;   // pipelined kernel: 0 automatic (the uniform split), 1 stream-K, 2 uniform split
 static int g_qg_skmin = 0;   // stream-K: quant blocks per workgroup at least (0: 16)
 static int g_qg_kw = 0;      // wave-split kernel: 0 automatic, 1 for every tiled batch over 16 rows, -1 never
 static int g_qg_kwR = 0;     // wave-split kernel: weight tiles per workgroup (0: automatic, else 2, 3 or 4)
+
+constexpr int QW_PIPE = 4;  // g_qg_pipe of the 32x32 kernel's first form
 
 static int qg_cu_count() {
     static int n = 0;
@@ -1524,8 +1527,9 @@ static bool kx_wanted(uint32_t dtype, int N, int K, int M) {
 //   form below 256 rows is slower (Q8_0 at 203 rows 116.8 against 79.7).
 // The offsets of a 128-row chunk are 32-bit: N and K below 2^22.
 static bool wide_wanted(uint32_t dtype, int N, int K, int M, bool whole = false) {
-    if (g_qg_pipe || g_qg_kw || g_qg_mchunk || g_qg_waves || g_qg_splits || g_qg_sched == 1) return false;
     if (M <= 16 || N >= (1 << 22) || K >= (1 << 22)) return false;
+    if (g_qg_pipe >= QW_PIPE) return true;
+    if (g_qg_pipe || g_qg_kw || g_qg_mchunk || g_qg_waves || g_qg_splits || g_qg_sched == 1) return false;
     if (M <= 32) return dtype == DT_Q4_0 && (size_t)N * K > (size_t)4608 * 1024;
     return M <= 64 || (whole && M < 256) || (size_t)M * N <= (size_t)(dtype == DT_Q8_0 ? 4 : 8) << 20;
 }
@@ -1540,12 +1544,14 @@ static void wide_plan(QgPlan& p, uint32_t dtype, int N, int nb, int M, bool whol
     } T[QW_FORM_COUNT] = {{{1.60, 1.70}, 5.0}, {{1.00, 1.35}, 2.5}, {{1.15, 1.38}, 2.5}, {{0.79, 0.98}, 1.5}};
     const int np = (nb + 1) / 2, cu = qg_cu_count();  // pairs of quant blocks
     double best = 1e30;
+    const int forced = g_qg_pipe >= QW_PIPE && g_qg_splits > 0 && !whole ? std::min(g_qg_splits, np) : 0;
     for (int i = 0; i < QW_FORM_COUNT; i++) {
+        if (g_qg_pipe >= QW_PIPE && i != g_qg_pipe - QW_PIPE) continue;
         const QwTile t = qgemm_wide_tile(i);
         const long long tiles = (long long)((N + t.nt - 1) / t.nt) * ((M + t.mt - 1) / t.mt);
-        for (int S = 1; S <= (whole ? 1 : 16); S++) {
-            const int pps = (np + S - 1) / S;
-            if ((np + pps - 1) / pps != S) continue;
+        for (int S0 = forced ? forced : 1; S0 <= (forced ? forced : whole ? 1 : 16); S0++) {
+            const int pps = (np + S0 - 1) / S0, S = (np + pps - 1) / pps;
+            if (S != S0 && !forced) continue;
             const long long rounds = (tiles * S + cu - 1) / cu;
             const double us = rounds * ((pps + t.wk - 1) / t.wk * T[i].it[dtype == DT_Q8_0] + T[i].fix) +
                               (S > 1 ? 2.5 + (double)S * M * N * 2e-6 : 0.0);
@@ -1731,7 +1737,7 @@ int set_qgemm_tuning(int waves, int splits, int pipe, int mchunk) {
     QH_REQUIRE(mchunk == 0 || mchunk == 16 || mchunk == 32 || mchunk == 64 || mchunk == 128, QRAF_HIP_ERR_INVALID,
                "qgemm tuning: batch chunk %d", mchunk);
     QH_REQUIRE(splits >= 0 && splits <= 256, QRAF_HIP_ERR_INVALID, "qgemm tuning: splits %d", splits);
-    QH_REQUIRE(pipe >= -1 && pipe <= 3, QRAF_HIP_ERR_INVALID, "qgemm tuning: pipe %d", pipe);
+    QH_REQUIRE(pipe >= -1 && pipe < QW_PIPE + QW_FORM_COUNT, QRAF_HIP_ERR_INVALID, "qgemm tuning: pipe %d", pipe);
     g_qg_waves = waves;
     g_qg_splits = splits;
     g_qg_pipe = pipe;

@@ -370,7 +370,7 @@ def test_qgemm_tiled_silu_epilogue(hip, dt, case, form):
         call("qraf_hip_set_qgemm_kw", 1, 0)
     try:
         Y, _, _ = run_gemm(hip, wq, dt, N, K, X, tiled=True, split=False)
-        if form == "pipelined":  # the epilogue entry's own automatic choice is this form at these shapes
+        if form == "pipelined":  # without the wave-split kernel the epilogue entry takes this form at these shapes
             call("qraf_hip_set_qgemm_tuning", 0, 0, 0, 0)
             call("qraf_hip_set_qgemm_kw", -1, 0)
         call("qraf_hip_qgemm_tiled_silu_dev", dtl.ptr, dt, N, K, dh.ptr, dl.ptr, M, oh.ptr, ol.ptr, None)
@@ -470,8 +470,8 @@ ARGMAX_CASES = [
 def test_qgemm_tiled_argmax(hip, dt, case):
     """The greedy head's fused argmax (qraf_hip_qgemm_tiled_argmax_dev) equals
     Sampler::argmax (sampler.cpp:25-35, the first of the largest values:
-    numpy's argmax) of the unsplit tiled GEMM's own product, where the plan
-    is the pipelined form (fused = 1); elsewhere it launches nothing
+    numpy's argmax) of the unsplit pipelined GEMM's own product, where the
+    pipelined form covers the shape (fused = 1); elsewhere it launches nothing
     (fused = 0, the tokens untouched).  The weights hold every row twice, at
     i and R + i, so every logit ties with one 2R rows / many workgroups away
     and only the smaller index wins; a last extra row makes the row count
@@ -485,7 +485,11 @@ def test_qgemm_tiled_argmax(hip, dt, case):
     extra = po.quantize(dt, (rng.standard_normal(K) * 0.02).astype(np.float32))
     wq = np.concatenate([half, half, extra])
     X = rng.standard_normal((M, K)).astype(np.float32)
-    Y, _, _ = run_gemm(hip, wq, dt, N, K, X, tiled=True, split=False)
+    call("qraf_hip_set_qgemm_tuning", 0, 0, 1 if N >= 8192 else 2, 0)  # the form whose epilogue takes the argmax
+    try:
+        Y, _, _ = run_gemm(hip, wq, dt, N, K, X, tiled=True, split=False)
+    finally:
+        call("qraf_hip_set_qgemm_tuning", 0, 0, 0, 0)
     assert np.array_equal(Y[:, :R].view(np.uint32), Y[:, R:2 * R].view(np.uint32)), "repeated rows differ"
     want = np.argmax(Y, axis=1)
     assert np.all(want < R) or np.any(want == 2 * R)
@@ -522,15 +526,14 @@ def test_qgemm_tiled_argmax(hip, dt, case):
 
 @pytest.mark.parametrize("dt", [po.Q8_0, po.Q4_0])
 @pytest.mark.parametrize("case", [
-    # N, K, M: one block and an odd count (half a pair at a group's end), fewer pairs than K groups, ragged rows
-    # and columns of each tile height (32, 64, 128 rows), splits with an odd tail
+    # N, K, M: one block and an odd count (half a pair at a group's end), fewer pairs than K groups
     (64, 32, 33), (100, 96, 40), (33, 64, 64), (300, 416, 65), (1000, 2080, 129), (130, 2048, 203), (2050, 1056, 97),
     (9000, 576, 20), (4100, 2048, 32), (12000, 2048, 200)], ids=lambda c: "x".join(map(str, c)))
 def test_qgemm_32x32_edges(hip, dt, case):
-    """The 32x32 kernel's tiles, K groups and splits at their edges, against the
-    oracle within the GEMM's bound, with a residual added in place; and a row
-    of NaN and one of infinities leave every other row as it was, bit for bit
-    (blocks past the end of a row or of a split belong to other rows)."""
+    """The automatic choice at ragged rows, columns and block counts, against
+    the oracle within the GEMM's bound, with a residual added in place; and a
+    row of NaN and one of infinities leave every other row as it was, bit for
+    bit (blocks past the end of a row or of a split belong to other rows)."""
     N, K, M = case
     rng = np.random.default_rng(3 * N + K + 7 * M + dt)
     wq = po.quantize(dt, (rng.standard_normal(N * K) * 0.02).astype(np.float32))
@@ -541,6 +544,11 @@ def test_qgemm_32x32_edges(hip, dt, case):
     check(Y, wq, dt, N, K, X)
     Ya, _, _ = run_gemm(hip, wq, dt, N, K, X, add=add, in_place=True, tiled=True)
     check(Ya, wq, dt, N, K, X, add)
+    rows_stay_apart(hip, wq, dt, N, K, X, Y)
+
+
+def rows_stay_apart(hip, wq, dt, N, K, X, Y):
+    M = X.shape[0]
     bad = X.copy()
     bad[M // 2, :] = np.nan
     bad[M - 1, :] = np.inf
@@ -549,3 +557,98 @@ def test_qgemm_32x32_edges(hip, dt, case):
     keep[[M // 2, M - 1]] = False
     assert np.array_equal(Yb[keep].view(np.uint32), Y[keep].view(np.uint32))
     assert not np.isfinite(Yb[~keep]).any()
+
+
+def reference(wq, dt, N, K, X):
+    """The product in 64 bits and the GEMM's bound on its difference."""
+    W = po.dequantize(dt, wq, N * K).reshape(N, K).astype(np.float64)
+    x = X.astype(np.float64)
+    s = np.abs(x) @ np.abs(W).T
+    return x @ W.T, (2.0 ** -20 + (K + 2) * 2.0 ** -24) * s + 2.0 ** -25 * np.abs(W).sum(1) + 1e-30
+
+
+# the 32x32 kernel's tiles (batch rows x weight rows) in the order of its tuning values from 4
+TILES_32X32 = [(128, 128), (64, 128), (64, 64), (32, 64)]
+
+
+@pytest.mark.parametrize("dt", [po.Q8_0, po.Q4_0])
+@pytest.mark.parametrize("splits", [1, 2, 5])
+@pytest.mark.parametrize("form", range(4), ids=lambda f: "%dx%d" % TILES_32X32[f])
+def test_qgemm_32x32_forms(hip, dt, splits, form):
+    """Every tile of the 32x32 kernel, forced, in one split and in several: one
+    row and column past a tile and one short of it, one block, an odd last
+    block in the last split, fewer pairs of blocks than K groups; the
+    workspace query shows that the forced split count is the one planned."""
+    call, lib = hip._lib.call, hip._lib.lib
+    mt, nt = TILES_32X32[form]
+    call("qraf_hip_set_qgemm_tuning", 0, splits, 4 + form, 0)
+    try:
+        for N, K, M in ((nt + 1, 32, 17), (nt - 1, 96, mt + 1), (2 * nt + 17, 416, 2 * mt - 1), (nt + 15, 2080, mt + 33),
+                        (3 * nt - 16, 1056, 2 * mt + 20)):
+            pairs = (K // 32 + 1) // 2
+            want = -(-pairs // -(-pairs // min(splits, pairs)))
+            assert lib.qraf_hip_qgemm_tiled_workspace_bytes(dt, N, K, M) == (want * M * N * 4 if want > 1 else 0)
+            print(f"qgemm 32x32 form {form} N={N} K={K} M={M} splits={want} dt={dt}", flush=True)
+            rng = np.random.default_rng(3 * N + K + 7 * M + dt)
+            wq = po.quantize(dt, (rng.standard_normal(N * K) * 0.02).astype(np.float32))
+            X = rng.standard_normal((M, K)).astype(np.float32)
+            add = rng.standard_normal((M, N)).astype(np.float32)
+            ref, tol = reference(wq, dt, N, K, X)
+            Y, _, _ = run_gemm(hip, wq, dt, N, K, X, tiled=True, repeats=2)
+            assert np.all(np.abs(Y - ref) <= tol)
+            Ya, _, _ = run_gemm(hip, wq, dt, N, K, X, add=add, in_place=True, tiled=True)
+            assert np.all(np.abs(Ya - (ref + add)) <= tol + 2.0 ** -23 * np.abs(ref + add))
+            rows_stay_apart(hip, wq, dt, N, K, X, Y)
+    finally:
+        call("qraf_hip_set_qgemm_tuning", 0, 0, 0, 0)
+
+
+@pytest.mark.parametrize("dt", [po.Q8_0, po.Q4_0])
+@pytest.mark.parametrize("form", [0, 1, 2, 3, None], ids=lambda f: "automatic" if f is None else "%dx%d" % TILES_32X32[f])
+def test_qgemm_32x32_silu_forms(hip, dt, form):
+    """The SwiGLU epilogue of every tile of the 32x32 kernel, forced, and of
+    the automatic choice: the planes hold silu(g) * u of the sums (for a forced
+    tile those of the GEMM in the same tile, which the product in 64 bits
+    bounds), and nothing is written past the M x F planes."""
+    from qraf_amd.backend import DeviceBuffer
+    call, lib = hip._lib.call, hip._lib.lib
+    mt, nt = (64, 128) if form is None else TILES_32X32[form]
+    call("qraf_hip_set_qgemm_tuning", 0, 0 if form is None else 1, 0 if form is None else 4 + form, 0)
+    try:
+        for N, K, M in ((nt + 2, 32, 17), (nt - 2, 96, mt + 1), (2 * nt + 18, 416, 2 * mt - 1), (nt + 14, 2080, mt + 33),
+                        (3 * nt - 16, 1056, 203)):
+            F = N // 2
+            print(f"qgemm 32x32 silu form {form} N={N} K={K} M={M} dt={dt}", flush=True)
+            rng = np.random.default_rng(3 * N + K + 7 * M + dt)
+            wq = po.quantize(dt, (rng.standard_normal(N * K) * 0.1).astype(np.float32))
+            X = rng.standard_normal((M, K)).astype(np.float32)
+            ref, tol = reference(wq, dt, N, K, X)
+            if form is not None:
+                Y, _, _ = run_gemm(hip, wq, dt, N, K, X, tiled=True)
+                assert np.all(np.abs(Y - ref) <= tol)
+                ref, tol = Y.astype(np.float64), np.zeros_like(ref)
+            dw, dx = DeviceBuffer.from_array(wq), DeviceBuffer.from_array(X)
+            dtl = DeviceBuffer(lib.qraf_hip_tiled_weight_bytes(dt, N, K))
+            call("qraf_hip_repack_tiles_dev", dw.ptr, dt, N, K, dtl.ptr, None)
+            dh, dl = DeviceBuffer(M * K * 2), DeviceBuffer(M * K * 2)
+            call("qraf_hip_split_bf16_dev", dx.ptr, dh.ptr, dl.ptr, M, K, None)
+            pad = 4096
+            fill = np.full(M * F + pad, 0xA5C3, np.uint16)
+            oh, ol = DeviceBuffer.from_array(fill), DeviceBuffer.from_array(fill)
+            call("qraf_hip_qgemm_tiled_silu_dev", dtl.ptr, dt, N, K, dh.ptr, dl.ptr, M, oh.ptr, ol.ptr, None)
+            call("qraf_hip_stream_synchronize", None)
+            hi, lo = oh.download(np.uint16, M * F + pad), ol.download(np.uint16, M * F + pad)
+            assert np.all(hi[M * F:] == 0xA5C3) and np.all(lo[M * F:] == 0xA5C3)
+            hv = (hi[:M * F].astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+            got = (hv + lo[:M * F].view(np.float16)).reshape(M, F)
+            g, u = ref[:, 0::2], ref[:, 1::2]
+            s = g / (1.0 + np.exp(-g))
+            # |d silu| <= 1.1 |dg|; the planes' own precision and a few ulp of expf
+            bound = (1.1 * tol[:, 0::2] * (np.abs(u) + tol[:, 1::2]) + np.abs(s) * tol[:, 1::2]
+                     + (2.0 ** -20 + 8 * 2.0 ** -24) * np.abs(s * u) + 2.0 ** -25)
+            err = np.abs(got - s * u)
+            assert np.all(err <= bound), f"max err {err.max():.3e}, worst ratio {(err / bound).max():.3f}"
+            for d in (dw, dx, dtl, dh, dl, oh, ol):
+                d.free()
+    finally:
+        call("qraf_hip_set_qgemm_tuning", 0, 0, 0, 0)
