@@ -1512,49 +1512,50 @@ static bool kx_wanted(uint32_t dtype, int N, int K, int M) {
     return (M > 32 && M <= 64 && N >= 16384) || (M > 64 && dtype == DT_Q8_0 && K >= 8192);
 }
 
-// Whether the 32x32 kernel (qgemm_wide.hip) takes a tiled N x K product of M
-// rows, unless a tuning call forces an older form.  Both sides measured on
-// MI355X over 20-512 rows of the Qwen2.5-3B, SmolLM2 and head shapes (GEMM and
-// partial sums, graph-timed); it is the faster one (1.05-2.8x) except
-//   17-32 rows of Q8_0 (2048 x 2048 7.8 against 9.2 us, 22016 x 2048 24.1 against
-//   23.4) and of small Q4_0 products (2048 x 2048 7.9 against 8.5; 2560 x 2048 is
-//   8.8 against 7.9), where a workgroup's start and end are most of its time;
-//   more than 64 rows of the largest outputs (Q4_0 22016 x 2048 at 384 rows 90.8
-//   against 102.9 us, at 256 rows 65.4 against 57.0; Q8_0 11008 x 2048 at 384 rows
-//   65.5 against 70.4, at 256 rows 44.7 against 36.6; the 151936-row head at 128
-//   rows ties): several full rounds of workgroups, where the older kernels' two
-//   workgroups per CU hide each other's start and end.  The SwiGLU entry's other
-//   form below 256 rows is slower (Q8_0 at 203 rows 116.8 against 79.7).
-// The offsets of a 128-row chunk are 32-bit: N and K below 2^22.
-static bool wide_wanted(uint32_t dtype, int N, int K, int M, bool whole = false) {
-    if (M <= 16 || N >= (1 << 22) || K >= (1 << 22)) return false;
-    if (g_qg_pipe >= QW_PIPE) return true;
-    if (g_qg_pipe || g_qg_kw || g_qg_mchunk || g_qg_waves || g_qg_splits || g_qg_sched == 1) return false;
-    if (M <= 32) return dtype == DT_Q4_0 && (size_t)N * K > (size_t)4608 * 1024;
-    return M <= 64 || (whole && M < 256) || (size_t)M * N <= (size_t)(dtype == DT_Q8_0 ? 4 : 8) << 20;
+static QgPlan qgemm_plan(uint32_t dtype, int N, int K, int M, size_t row_bytes, bool tiled, bool wide = true);
+
+// Rounds of W workgroups over `slots` resident ones; a last round takes `part`
+// of a full one's time however few workgroups it has, and more with its fill.
+static double qg_rounds(long long W, int slots, double part) {
+    const long long rem = W % slots;
+    return (double)(W / slots) + (rem ? part + (1 - part) * (double)rem / slots : 0.0);
 }
 
-// The wide kernel's form and split count: the least rounds of workgroups (one
-// per CU) x (iterations x us each + us to start and finish), plus the launch and
-// the traffic of the partial slices.  The us were fitted to each form's time
-// over K (MI355X: 256 rows of weights, one round, K = 4096 and 8192).
-static void wide_plan(QgPlan& p, uint32_t dtype, int N, int nb, int M, bool whole) {
+// The wide kernel's form and split count: the least modelled time (us), which
+// is returned.  Rounds of workgroups (one per CU; the Q4_0 64 x 128 tile leaves
+// room for two, which then share the CU) x (us an iteration of WK pairs of
+// blocks x iterations + us to start and finish, longer for the SwiGLU epilogue)
+// + the launch + the traffic of the partial slices.  Fitted to 43,000 timings of
+// every form and split on MI355X (17-1,024 rows, N 576-151936, K 256-18944):
+// median error 2-5%; the plan it picks is 0.3% off the best of them on average.
+static double wide_plan(QgPlan& p, uint32_t dtype, int N, int nb, int M, bool whole) {
     static constexpr struct {
-        double it[2], fix;  // Q4_0, Q8_0
-    } T[QW_FORM_COUNT] = {{{1.60, 1.70}, 5.0}, {{1.00, 1.35}, 2.5}, {{1.15, 1.38}, 2.5}, {{0.79, 0.98}, 1.5}};
-    const int np = (nb + 1) / 2, cu = qg_cu_count();  // pairs of quant blocks
+        double it[2], fix[2], fix_silu[2], launch;  // Q4_0, Q8_0
+    } T[QW_FORM_COUNT] = {{{1.62, 1.74}, {3.8, 3.8}, {9.5, 9.5}, 2.4},
+                          {{1.10, 1.31}, {0.5, 3.0}, {2.4, 5.6}, 2.0},
+                          {{1.25, 1.43}, {2.8, 2.8}, {3.9, 3.9}, 1.7},
+                          {{0.80, 0.94}, {2.4, 2.4}, {2.9, 2.9}, 1.9}};
+    const int np = (nb + 1) / 2, cu = qg_cu_count(), q8 = dtype == DT_Q8_0;  // np: pairs of quant blocks
     double best = 1e30;
     const int forced = g_qg_pipe >= QW_PIPE && g_qg_splits > 0 && !whole ? std::min(g_qg_splits, np) : 0;
     for (int i = 0; i < QW_FORM_COUNT; i++) {
         if (g_qg_pipe >= QW_PIPE && i != g_qg_pipe - QW_PIPE) continue;
         const QwTile t = qgemm_wide_tile(i);
+        const double fix = whole ? T[i].fix_silu[q8] : T[i].fix[q8];
         const long long tiles = (long long)((N + t.nt - 1) / t.nt) * ((M + t.mt - 1) / t.mt);
         for (int S0 = forced ? forced : 1; S0 <= (forced ? forced : whole ? 1 : 16); S0++) {
             const int pps = (np + S0 - 1) / S0, S = (np + pps - 1) / pps;
             if (S != S0 && !forced) continue;
-            const long long rounds = (tiles * S + cu - 1) / cu;
-            const double us = rounds * ((pps + t.wk - 1) / t.wk * T[i].it[dtype == DT_Q8_0] + T[i].fix) +
-                              (S > 1 ? 2.5 + (double)S * M * N * 2e-6 : 0.0);
+            const long long W = tiles * S;
+            const int n = (pps + t.wk - 1) / t.wk;
+            double us = S > 1 ? 1.0 + 0.25 * S + (double)S * M * N * 1.5e-6 : 0.0;
+            if (i == 1 && !q8) {
+                const double one = n * T[i].it[0] + fix, two = n * 1.68 + fix + 1.5;
+                const long long rem = W % (2 * cu);
+                us += (double)(W / (2 * cu)) * two + (rem > cu ? two : rem ? one : 0.0) + 4.3;
+            } else {
+                us += qg_rounds(W, cu, 1.0) * (n * T[i].it[q8] + fix) + T[i].launch;
+            }
             if (us < best) {
                 best = us;
                 p.wide = i + 1;
@@ -1568,15 +1569,89 @@ static void wide_plan(QgPlan& p, uint32_t dtype, int N, int nb, int M, bool whol
         }
     }
     p.ws_bytes = p.S > 1 ? (size_t)p.S * M * N * 4 : 0;
+    return best;
+}
+
+// Modelled time (us) of the older forms where they compete with the 32x32
+// kernel: over 64 rows, and 33-64 rows of at least 16384 weight rows (whole: the
+// SwiGLU entry's unsplit form below 256 rows).  Rounds of workgroups x (us a
+// quant block x blocks + us to start and finish) + the launch + the partial
+// slices; fitted as above (median error 2-5%).
+static double older_us(uint32_t dtype, int N, int K, int M, bool whole) {
+    struct Cost {
+        int slots;
+        double block, fix, launch, part;
+    };
+    const int q8 = dtype == DT_Q8_0, nb = K / 32, cu = qg_cu_count();
+    if (whole) {  // narrow pipelined form, 128 weight x 64 batch rows
+        const Cost c = q8 ? Cost{cu, 0.518, 4.05, 2.5, 1.0} : Cost{2 * cu, 0.544, 4.1, 2.9, 0.8};
+        return qg_rounds((long long)((N + 127) / 128) * ((M + 63) / 64), c.slots, c.part) *
+                   ((nb + 1) / 2 * 2 * c.block + c.fix) + c.launch;
+    }
+    const QgPlan p = qgemm_plan(dtype, N, K, M, q_row_bytes(dtype, 32, K), true, false);
+    Cost c;
+    if (p.kxT == 4) c = q8 ? Cost{2 * cu, 0.838, 6.6, 0.8, 0.52} : Cost{2 * cu, 0.858, 5.3, 1.7, 0.48};
+    else if (p.kxT) c = Cost{2 * cu, 1.245, 0.3, 9.7, 1.0};
+    else if (p.pipe && p.WN == 4) c = q8 ? Cost{cu, 0.50, 2.5, 2.8, 1.0} : Cost{2 * cu, 0.60, 3.4, 2.5, 0.68};
+    else if (p.pipe && p.TN == 3) c = Cost{cu, 1.21, 9.2, 1.6, 1.0};
+    else if (p.pipe) c = q8 ? Cost{cu, 0.87, 6.1, 2.6, 1.0} : Cost{cu, 0.89, 5.8, 2.4, 1.0};
+    else c = q8 ? Cost{cu, 0.289, 4.6, 0.0, 0.92} : Cost{cu, 0.336, 5.0, 0.0, 0.92};
+    return qg_rounds((long long)p.ntiles * p.mchunks * p.S, c.slots, c.part) * (p.bps * c.block + c.fix) + c.launch +
+           (p.S > 1 ? 2.0 + (double)p.S * M * N * 1.4e-6 : 0.0);
+}
+
+// Whether the 32x32 kernel (qgemm_wide.hip) takes a tiled N x K product of M
+// rows (whole: with the SwiGLU epilogue), and then its plan, unless a tuning
+// call forces an older form.  Both sides timed on MI355X over the ranges above:
+//   over 64 rows, outputs of up to 8M (Q4_0) or 4M (Q8_0) elements: the modelled
+//   times decide, the 32x32 kernel where it leads by 5%, about their error (Q4_0 22016 x 2048 at 128
+//   rows 42.9 against 37.3 us; 49152 x 576 at 160 rows 30.6 against 33.8; Q8_0 2048 x
+//   11008 at 203 rows 52.1 against 33.6).  Beyond (Q4_0 22016 x 2048 at 384 rows 90.8
+//   against 102.9) several full rounds of the older kernels, two workgroups per
+//   CU, hide each other's start and end;
+//   33-64 rows from 16384 weight rows on: as modelled, by 10%; Q8_0 stays with the
+//   row-split kernel in most of that range (49152 x 576 at 64 rows 16.1 against 23.6,
+//   151936 x 2048 111 against 125);
+//   33-64 rows below that: the 32x32 kernel (Q4_0 11008 x 2048 at 64 rows 21.9
+//   against 14.4) except, for Q8_0 up to 40 rows, products with few blocks or more
+//   than 8192 weight rows (the wave-split kernel's chunk is half empty: 9728 x 896
+//   at 33 rows 8.6 against 9.7, at 48 11.2 against 10.8) and the SwiGLU entry's
+//   shortest ones;
+//   17-32 rows: Q4_0 products of more than 4.6M weights (11008 x 2048 at 32 rows 14.2
+//   against 10.8, 2560 x 2048 8.8 against 7.9, 2048 x 2048 7.9 against 8.5; Q8_0 2048
+//   x 2048 7.8 against 9.2);
+//   the SwiGLU entry: below 256 rows as modelled (Q8_0 22016 x 2048 at 203 rows 116.8
+//   against 79.7; Q4_0 16384 x 256 at 160 rows 11.2 against 14.7), from 256 rows within
+//   the limit above (Q4_0 8192 x 2048 at 512 rows 68.1 against 38.7), its short
+//   products at 17-20 rows not (5120 x 960 at 17 rows 7.1 against 7.8).
+// The offsets of a 128-row chunk are 32-bit: N and K below 2^22.
+static bool wide_wanted(QgPlan& p, uint32_t dtype, int N, int K, int M, bool whole) {
+    if (M <= 16 || N >= (1 << 22) || K >= (1 << 22)) return false;
+    const bool q8 = dtype == DT_Q8_0;
+    bool wanted = true, model = false;
+    if (g_qg_pipe >= QW_PIPE) wanted = true;
+    else if (g_qg_pipe || g_qg_kw || g_qg_mchunk || g_qg_waves || g_qg_splits || g_qg_sched == 1) wanted = false;
+    else if (M <= 32)
+        wanted = !q8 && (size_t)N * K > (size_t)4608 * 1024 && !(whole && (K < 640 ? M <= 28 : M <= 20 && K < 1280));
+    else if (M > 64 && (!whole || M >= 256) && (size_t)M * N > (size_t)(q8 ? 4 : 8) << 20) wanted = false;
+    else if (whole && M >= 256) wanted = true;
+    else if (M <= 64 && N < 16384)
+        wanted = q8 ? M <= 40 ? K >= (whole ? 640 : 512) && N <= 8192
+                              : !whole || M > 56 || (K >= 512 && (N <= 8192 || K >= 1024 || M > 48))
+                    : !whole || M > 40 || K >= 640 || (K >= 512 && N <= 8192);
+    else model = true;
+    if (!wanted) return false;
+    QgPlan w{};
+    const double us = wide_plan(w, dtype, N, K / 32, M, whole);
+    if (model && us >= (M > 64 ? 0.95 : 0.9) * older_us(dtype, N, K, M, whole)) return false;
+    p = w;
+    return true;
 }
 
 // wide: the 32x32 kernel may be the plan (the argmax epilogue exists in the pipelined one only)
-static QgPlan qgemm_plan(uint32_t dtype, int N, int K, int M, size_t row_bytes, bool tiled, bool wide = true) {
+static QgPlan qgemm_plan(uint32_t dtype, int N, int K, int M, size_t row_bytes, bool tiled, bool wide) {
     QgPlan p{};
-    if (tiled && wide && wide_wanted(dtype, N, K, M)) {
-        wide_plan(p, dtype, N, K / 32, M, false);
-        return p;
-    }
+    if (tiled && wide && wide_wanted(p, dtype, N, K, M, false)) return p;
     if (tiled && kx_wanted(dtype, N, K, M)) {
         kx_plan(p, N, K / 32, M, false);
         return p;
@@ -2091,11 +2166,8 @@ int launch_qgemm_silu(const void* Wt, uint32_t dtype, int N, int K, const uint16
     QH_REQUIRE(((((uintptr_t)Wt) | ((uintptr_t)xh) | ((uintptr_t)xl)) & 15) == 0, QRAF_HIP_ERR_INVALID,
                "qgemm silu: misaligned operands");
     const int nb = K / 32, KC = 2;
-    if (wide_wanted(dtype, N, K, M, true)) {
-        QgPlan p{};
-        wide_plan(p, dtype, N, nb, M, true);
+    if (QgPlan p{}; wide_wanted(p, dtype, N, K, M, true))
         return launch_qgemm_wide(p.wide - 1, Wt, dtype, N, K, xh, xl, M, nullptr, nullptr, 1, p.bps, act_hi, act_lo, s);
-    }
     if (g_qg_pipe == 3 ? M > 16 : (g_qg_pipe == 0 && g_qg_kw == 0 && M >= 256)) {
         QgPlan p{};
         kx_plan(p, N, nb, M, true);

@@ -603,6 +603,34 @@ def test_qgemm_32x32_forms(hip, dt, splits, form):
         call("qraf_hip_set_qgemm_tuning", 0, 0, 0, 0)
 
 
+@pytest.mark.parametrize("dt,N,K,M,form", [
+    # tuning (pipe value, wave-split mode) of the kernel that the default must be: row-split, wave-split, pipelined
+    (po.Q8_0, 49152, 576, 64, (3, 0)), (po.Q8_0, 49152, 2048, 33, (3, 0)), (po.Q8_0, 9728, 896, 33, (0, 1)),
+    (po.Q4_0, 49152, 576, 160, (1, 0)), (po.Q8_0, 49152, 576, 80, (1, 0)),
+    # and of the 32x32 kernel's tiles
+    (po.Q4_0, 22016, 2048, 160, (5, 0)), (po.Q4_0, 11008, 4096, 96, (5, 0)), (po.Q4_0, 22016, 2048, 128, (4, 0)),
+    (po.Q8_0, 8192, 1024, 48, (7, 0))], ids=lambda v: str(v).replace(" ", ""))
+def test_qgemm_default_form(hip, dt, N, K, M, form):
+    """The default of these products is the kernel that measured faster there:
+    its result equals that kernel's, forced, bit for bit, in the same splits."""
+    call, lib = hip._lib.call, hip._lib.lib
+    rng = np.random.default_rng(N + M)
+    one = po.quantize(dt, (rng.standard_normal(97 * K) * 0.02).astype(np.float32))
+    wq = np.resize(one, one.size // 97 * N)  # the 97 rows over and over
+    X = rng.standard_normal((M, K)).astype(np.float32)
+    slices = lib.qraf_hip_qgemm_tiled_workspace_bytes(dt, N, K, M) // (M * N * 4) or 1
+    print(f"qgemm default form N={N} K={K} M={M} dt={dt} slices={slices}", flush=True)
+    Y, _, _ = run_gemm(hip, wq, dt, N, K, X, tiled=True)
+    call("qraf_hip_set_qgemm_tuning", 0, slices, form[0], 0)
+    call("qraf_hip_set_qgemm_kw", form[1], 0)
+    try:
+        Yf, _, _ = run_gemm(hip, wq, dt, N, K, X, tiled=True)
+    finally:
+        call("qraf_hip_set_qgemm_tuning", 0, 0, 0, 0)
+        call("qraf_hip_set_qgemm_kw", 0, 0)
+    assert np.array_equal(Y.view(np.uint32), Yf.view(np.uint32))
+
+
 @pytest.mark.parametrize("dt", [po.Q8_0, po.Q4_0])
 @pytest.mark.parametrize("form", [0, 1, 2, 3, None], ids=lambda f: "automatic" if f is None else "%dx%d" % TILES_32X32[f])
 def test_qgemm_32x32_silu_forms(hip, dt, form):
