@@ -535,7 +535,8 @@ __global__ __launch_bounds__(SNT) void sample_rows_kernel(const float* __restric
             lo = fminf(lo, s_red[1][w]);
         }
         __syncthreads();  // s_red may be written again
-        if (lo > -INFINITY && hi < INFINITY) {
+        // (p infinite: its ties span logits below the bound, and go by index)
+        if (lo / T > -INFINITY && hi / T < INFINITY) {
             // #{maxima >= lo} = clo >= cutoff throughout
             int clo = NSUB * SNT;
             const int target = cutoff + (cutoff >> 2) + 8;

@@ -65,3 +65,22 @@ def test_sampling_with_sub_range_maxima(hip, V, k):
         got, _ = device_sample(hip, L, (T, k, top_p, 1.0), uniforms=np.array(uni, np.float32))
         for kind, (g, w) in enumerate(zip(got, want)):
             assert w is None or g == w, f"V={V} k={k} T={T} top_p={top_p} kind={kind}: {g} against {w}"
+
+
+@pytest.mark.parametrize("V", [16448, 151936])
+@pytest.mark.parametrize("k", [1, 40, 100])
+def test_temperatures_that_overflow(hip, V, k):
+    """logit / T past the range of fp32: every such p is the same infinity, the
+    candidates are those of the lowest index, their exponentials NaN, and the
+    token the last candidate (no sum reaches top_p or the uniform)."""
+    rng = np.random.default_rng(V + k)
+    L = (rng.standard_normal((5, V)) * 2).astype(np.float32)
+    L[1] -= 1000  # every p is -inf
+    L[2] = np.round(L[2])
+    L[3, : V // 2] -= 50
+    L[4] *= np.float32(1e3)
+    for top_p in (0.9, 1.0):
+        with np.errstate(over="ignore", invalid="ignore"):
+            want = [candidates(l, 1e-38, k, top_p)[0][-1] for l in L]
+        got, _ = device_sample(hip, L, (1e-38, k, top_p, 1.0), uniforms=np.full(5, 0.5, np.float32))
+        assert list(got) == want, f"V={V} k={k} top_p={top_p}"
