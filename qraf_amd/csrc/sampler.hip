@@ -426,6 +426,12 @@ __global__ __launch_bounds__(SNT) void sample_rows_kernel(const float* __restric
     int nsort = cutoff;
     bool fast = cutoff == V;  // every token a candidate
     bool gathered = false;    // the candidates are in cval / cidx
+    // what the sub-range maxima leave to the search: a part of the row that holds
+    // the candidates (from a bound that cut_n values reach to the largest), or, as
+    // some p is infinite, nothing
+    int cut_n = V;
+    float cut_lo = -INFINITY, cut_hi = INFINITY;
+    bool infinite = false;
     float t = -INFINITY;
     // the row's sort storage: pairs (pa, ia), the radix sort's other buffer (pb, ib)
     float* pa = sort_ws + (size_t)row * 4 * V;
@@ -495,7 +501,8 @@ __global__ __launch_bounds__(SNT) void sample_rows_kernel(const float* __restric
     // comment).  Bound by the row's bytes (one workgroup per row; the search passes
     // below read the row once each): MI355X, 128 rows x 151936, top-k 40, top-p 0.9:
     // 114 -> 28 us (77.8 MB read once: 15 us at the rate of a large copy).  Left
-    // to the searches below: maxima that are not finite (masked rows) and more than CAND_CAP values at the bound.
+    // to the searches below: maxima that are not finite (masked rows) and more
+    // than CAND_CAP values at the bound.
     if (!fast && !big && (V & 3) == 0 && V >= SUB_MIN && cutoff <= SUB_CUT) {
         const float4* l4 = (const float4*)l;
         const int V4 = V >> 2, Q = (V4 + NSUB - 1) / NSUB;  // float4s per sub-range
@@ -546,7 +553,8 @@ __global__ __launch_bounds__(SNT) void sample_rows_kernel(const float* __restric
                 int mine = 0;
 #pragma unroll
                 for (int j = 0; j < 8; j++) {
-                    th[j] = lo + (hi - lo) * ((float)(j + 1) / 9.0f);
+                    // the fourth pass counts the maxima equal to the largest (rows of few values)
+                    th[j] = pass == 3 && j == 7 ? hi : lo + (hi - lo) * ((float)(j + 1) / 9.0f);
                     int c = 0;
 #pragma unroll
                     for (int q = 0; q < NSUB; q++) c += __popcll(__ballot(mx[q] >= th[j]));
@@ -580,6 +588,7 @@ __global__ __launch_bounds__(SNT) void sample_rows_kernel(const float* __restric
 #pragma unroll
             for (int q = 0; q < NSUB; q++) {
                 if (!(mx[q] >= tg)) continue;
+                if (q && *(volatile int*)&s_n > CAND_CAP) break;  // given up: the search takes the row
                 const int b1 = min(V4, (q + 1) * Q);
                 for (int base = q * Q + tid; base < b1; base += SNT * 5) {
                     float4 v[5];
@@ -606,7 +615,19 @@ __global__ __launch_bounds__(SNT) void sample_rows_kernel(const float* __restric
             __syncthreads();
             gathered = s_n <= CAND_CAP;
             if (gathered) nsort = s_n;
+            else {
+                cut_n = CAND_CAP + 1;
+                cut_lo = lo / T;
+                cut_hi = hi / T;
+            }
             __syncthreads();  // s_n may be written again
+        } else {
+            // a sub-range without a number above -inf: masked, or of NaN (then unknown)
+            bool masked = false;
+#pragma unroll
+            for (int q = 0; q < NSUB; q++)
+                if (mx[q] == -INFINITY) masked |= l[4 * (q * Q + tid)] == -INFINITY;
+            infinite = __syncthreads_or(masked || hi / T == INFINITY || (lo > -INFINITY && lo / T == -INFINITY));
         }
     }
     if (gathered && nsort <= 64) {
@@ -619,31 +640,35 @@ __global__ __launch_bounds__(SNT) void sample_rows_kernel(const float* __restric
     // 8-way search between the row's smallest and largest p; then every
     // p >= t is gathered and sorted.  The sort makes the result independent
     // of the gather order, and equal to the radix path's.
-    if (!fast && !big && !gathered) {
-        float mx = -INFINITY, mn = INFINITY;
-        for_row(l, V, tid, [&](int, float v) {
-            const float p = v / T;
-            mx = fmaxf(mx, p);
-            mn = fminf(mn, p);
-        });
+    if (!fast && !big && !gathered && !infinite) {
+        float mx = cut_hi, mn = cut_lo;
+        if (cut_n == V) {
+            mx = -INFINITY;
+            mn = INFINITY;
+            for_row(l, V, tid, [&](int, float v) {
+                const float p = v / T;
+                mx = fmaxf(mx, p);
+                mn = fminf(mn, p);
+            });
 #pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) {
-            mx = fmaxf(mx, __shfl_xor(mx, o));
-            mn = fminf(mn, __shfl_xor(mn, o));
-        }
-        if ((tid & 63) == 0) {
-            s_red[0][tid >> 6] = mx;
-            s_red[1][tid >> 6] = mn;
-        }
-        __syncthreads();
-        for (int w = 0; w < NW; w++) {
-            mx = fmaxf(mx, s_red[0][w]);
-            mn = fminf(mn, s_red[1][w]);
+            for (int o = 32; o >= 1; o >>= 1) {
+                mx = fmaxf(mx, __shfl_xor(mx, o));
+                mn = fminf(mn, __shfl_xor(mn, o));
+            }
+            if ((tid & 63) == 0) {
+                s_red[0][tid >> 6] = mx;
+                s_red[1][tid >> 6] = mn;
+            }
+            __syncthreads();
+            for (int w = 0; w < NW; w++) {
+                mx = fmaxf(mx, s_red[0][w]);
+                mn = fminf(mn, s_red[1][w]);
+            }
         }
         const int target = max(2 * cutoff, 512);
         if (mx > mn && mx < INFINITY && mn > -INFINITY) {
-            float lo = mn, hi = mx;  // #{p >= lo} = V >= cutoff
-            int clo = V;
+            float lo = mn, hi = mx;  // #{p >= lo} >= cutoff
+            int clo = cut_n;
             for (int pass = 0; pass < 16 && clo > target; pass++) {
                 float th[8];
 #pragma unroll

@@ -67,6 +67,44 @@ def test_sampling_with_sub_range_maxima(hip, V, k):
             assert w is None or g == w, f"V={V} k={k} T={T} top_p={top_p} kind={kind}: {g} against {w}"
 
 
+@pytest.mark.parametrize("V", [16448, 40000, 151936])
+@pytest.mark.parametrize("k", [1, 40, 100, 512])
+def test_rows_left_to_the_search(hip, V, k):
+    """Rows whose sub-range maxima are not finite or whose bound more than 4,096
+    values reach go to the search, or to the radix select, with what the first
+    read of the row found."""
+    rng = np.random.default_rng(V * k)
+    base = (rng.standard_normal(V) * 2).astype(np.float32)
+    rows = [base.copy() for _ in range(9)]
+    rows[0][V // 2:] = -np.inf          # a constrained vocabulary
+    rows[1][700:] = -np.inf
+    rows[2][5:4105] = -np.inf           # a sub-range of some threads only
+    rows[3] = np.minimum(base, 2.0)     # a sixth of the row equal, at the top
+    rows[4][:] = 1.5
+    rows[5] = np.where(rng.random(V) < 0.3, 5.0, -1.0)
+    rows[6][:5000] += 20                # more than 4,096 above the rest, all distinct
+    rows[7] = np.round(base * 2) / 2
+    rows[8][11] = np.inf                # its p - max is NaN: the last candidate
+    rows = [r.astype(np.float32) for r in rows]
+    for T, top_p in ((0.8, 0.9), (2.0, 1.0)):
+        want, uni = [], []
+        for i, l in enumerate(rows):
+            with np.errstate(invalid="ignore"):
+                o, cs = candidates(l, T, k, top_p)
+            r = np.float32(rng.random())
+            if not np.isfinite(cs).all():
+                want.append(o[-1])
+            else:
+                j = min(int(np.searchsorted(cs, r)), cs.size - 1)
+                if np.abs(cs - r).min() < 1e-5:
+                    r = np.float32(((float(cs[j - 1]) if j else 0.0) + float(cs[j])) / 2)
+                want.append(pick(o, cs, r) if np.abs(cs - r).min() >= 1e-6 else None)
+            uni.append(r)
+        got, _ = device_sample(hip, np.stack(rows), (T, k, top_p, 1.0), uniforms=np.array(uni, np.float32))
+        for i, (g, w) in enumerate(zip(got, want)):
+            assert w is None or g == w, f"V={V} k={k} T={T} row {i}: {g} against {w}"
+
+
 @pytest.mark.parametrize("V", [16448, 151936])
 @pytest.mark.parametrize("k", [1, 40, 100])
 def test_temperatures_that_overflow(hip, V, k):
