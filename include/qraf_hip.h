@@ -313,10 +313,12 @@ int qraf_hip_qgemm_tiled_dev(const void* w_tiled, uint32_t dtype, uint32_t out_d
                              const uint16_t* x_hi, const uint16_t* x_lo, int32_t batch, float* y, const float* add,
                              void* workspace, uint64_t workspace_bytes, void* stream);
 /* Greedy LM head without logits: tokens[b] = Sampler::argmax
- * (sampler.cpp:25-35: the first of the largest values) of row b of
- * qraf_hip_qgemm_tiled_dev's product (out_dim = vocabulary rows), the product
- * never written.  Where the tiled plan for this shape is the pipelined kernel
- * it runs unsplit, each workgroup writing its best (value, index) per row to
+ * (sampler.cpp:25-35: the first of the largest values) of row b of the
+ * product (out_dim = vocabulary rows), the product never written.  Where the
+ * pipelined kernel covers the shape (over 64 rows, 33-64 of wide products) it
+ * runs unsplit, also where qraf_hip_qgemm_tiled_dev would run another form
+ * (whose sums may order near ties differently), each workgroup writing its
+ * best (value, index) per row to
  * keys (8-byte aligned, at least qraf_hip_qgemm_tiled_argmax_keys_bytes), and
  * a second launch reduces them: *fused = 1.  Otherwise nothing is launched
  * and *fused = 0 (the caller then takes the argmax of the written product).
@@ -480,12 +482,14 @@ int qraf_engine_step_collect(qraf_engine* engine, uint32_t* next_tokens, int32_t
  * reference counterpart: an execution detail of qraf_engine_step. */
 int qraf_engine_set_graphs(qraf_engine* engine, int32_t on);
 /* keep = 0: a step that wants only greedy tokens (qraf_engine_step with
- * logits NULL and next_tokens set, qraf_engine_step_async) writes no logits:
- * where its head runs as the pipelined tile-major GEMM (more than 64 logit
- * rows at the usual vocabulary sizes) Sampler::argmax (sampler.cpp:25-35) is
- * taken in that GEMM's epilogue (qraf_hip_qgemm_tiled_argmax_dev), the same
- * tokens without the [rows][vocab] write and re-read; qraf_engine_sample and
- * qraf_engine_read_logits return QRAF_HIP_ERR_STATE after such a step.
+ * logits NULL and next_tokens set, qraf_engine_step_async) need not write
+ * logits: where its head's projection runs as the pipelined tile-major GEMM
+ * in one split (more than 64 logit rows of the largest vocabularies)
+ * Sampler::argmax (sampler.cpp:25-35) is taken in that GEMM's epilogue
+ * (qraf_hip_qgemm_tiled_argmax_dev), the same tokens without the
+ * [rows][vocab] write and re-read; qraf_engine_sample and
+ * qraf_engine_read_logits return QRAF_HIP_ERR_STATE after such a step,
+ * fused or not.
  * keep = 1 (the default): every step leaves its logits in HBM.  No reference
  * counterpart: the reference's forward always returns the logits. */
 int qraf_engine_set_keep_logits(qraf_engine* engine, int32_t keep);

@@ -1304,7 +1304,7 @@ static int step_issue(qraf_engine* e, int32_t n, const int32_t* seq_ids, const u
                                    c.rms_norm_eps, e->xhead, d_lrows);
                 if (argmax_only && dt != DT_F32 && e->head_t && !use_bmv(dt, V, D, n_logit_rows) &&
                     qgemm_argmax_fits(dt, V, D, n_logit_rows, e->am_keys_bytes)) {
-                    // the GEMM proj would run, with Sampler::argmax in its epilogue
+                    // the kernel proj would run, unsplit, with Sampler::argmax in its epilogue
                     QH_TRY(launch_split_bf16(e->xhead, e->xh, e->xl, n_logit_rows, D, 0, nullptr, s));
                     bool done = false;
                     QH_TRY(launch_qgemm_argmax(e->head_t, dt, V, D, e->xh, e->xl, n_logit_rows, e->am_keys,

@@ -2128,9 +2128,16 @@ static bool argmax_plan(uint32_t dtype, int N, int K, int M, size_t keys_bytes, 
     return p.mchunks <= 65535 && keys_bytes >= (size_t)p.ntiles * M * 8;
 }
 
+// Whether the fused head fits and launch_qgemm would run its kernel, unsplit:
+// else the engine writes the logits and takes their argmax, since sums in another
+// order may order near ties differently, and where the 32x32 kernel runs or the
+// product is split that is also faster (MI355X, 128 rows, argmax included: Q4_0
+// 32000 x 2048 45 us against 93 fused, Q8_0 50 against 76).
 bool qgemm_argmax_fits(uint32_t dtype, int N, int K, int M, size_t keys_bytes) {
     QgPlan p;
-    return argmax_plan(dtype, N, K, M, keys_bytes, p);
+    if (!argmax_plan(dtype, N, K, M, keys_bytes, p)) return false;
+    const QgPlan d = qgemm_plan(dtype, N, K, M, q_row_bytes(dtype, 32, K), true);
+    return !d.wide && d.S == 1;
 }
 
 int launch_qgemm_argmax(const void* Wt, uint32_t dtype, int N, int K, const uint16_t* xh, const uint16_t* xl, int M,

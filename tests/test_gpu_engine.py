@@ -967,3 +967,50 @@ def test_gemm_tuning_after_creation(hip):
         call("qraf_hip_set_qgemm_tuning", 0, 0, 0, 0)
         call("qraf_hip_set_qgemm_schedule", 0, 0)
         e.close()
+
+
+def test_greedy_only_head_near_ties(hip):
+    """keep_logits on and off give the same tokens where thousands of logits
+    differ only by the rounding of their sums.  Head rows hold one set of block
+    scales in every order, over blocks of equal quants; the rows' inputs repeat
+    in every block, so each row's logits are mathematically equal and its argmax
+    depends on the order in which the head's kernel adds the blocks."""
+    from itertools import islice, permutations
+
+    from qraf_amd.engine import Engine
+    V, D = 16385, 256
+    kw = dict(vocab=V, hidden=D, layers=1, heads=4, kv_heads=2, inter=512, max_seq=64, wdtype=po.Q4_0)
+    m = oracle_model(kw, 3)
+    rng = np.random.default_rng(8)
+    perms = np.array(list(islice(permutations(range(D // 32)), V)))
+    scales = (0.01 * (1 + rng.random(D // 32))).astype(np.float16)
+    head = np.zeros((V, D // 32, 18), np.uint8)
+    head[:, :, :2] = scales[perms].view(np.uint8).reshape(V, D // 32, 2)
+    head[:, :, 2:] = rng.integers(0, 256, 16, dtype=np.uint8)
+    emb = np.tile(rng.standard_normal((V, 32)).astype(np.float32), (1, D // 32))
+    e = Engine(engine_config(kw), kv_dtype=po.F32, max_batch=128)
+    try:
+        for name, dt, shape, data in m.tensors():
+            if "lm_head" in name:
+                data = head.reshape(-1)
+            elif "embed_tokens" in name:
+                data = po.quantize(dt, emb.reshape(-1))
+            elif "o_proj" in name or "down_proj" in name:
+                data = np.zeros_like(data)  # the layer adds nothing
+            e.set_tensor(name, dt, shape, data)
+        e.finalize()
+        for rows in (65, 96, 128):
+            print(f"greedy-only head at near ties, {rows} rows", flush=True)
+            toks = [int(t) for t in rng.integers(0, V, rows)]
+            got = []
+            for keep in (True, False):
+                e.set_keep_logits(keep)
+                seqs = [e.seq_create() for _ in range(rows)]
+                _, nx = e.step(seqs, toks, [0] * rows, logits=False, argmax=True)
+                got.append(nx.copy())
+                for s in seqs:
+                    e.seq_release(s)
+            assert len(set(got[0].tolist())) > 1
+            assert np.array_equal(got[0], got[1]), f"{rows} rows: {np.sum(got[0] != got[1])} tokens differ"
+    finally:
+        e.close()
