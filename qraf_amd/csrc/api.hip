@@ -56,6 +56,28 @@ hipStream_t default_stream() {
     return stream_of_current(&s) == QRAF_HIP_OK ? s : nullptr;
 }
 
+// A copy complete on return, ordered on the legacy stream as hipMemcpy's.  That
+// call (and hipMemset, hipDeviceSynchronize) fails while another thread captures
+// a stream, and breaks its capture; naming the stream does not.  A thread that
+// captures itself is refused, as before.
+static thread_local int t_captures = 0;  // begun by this thread's qraf_hip_graph_begin
+static int not_capturing() {
+    QH_REQUIRE(t_captures == 0, QRAF_HIP_ERR_HIP, "not permitted while this thread captures a graph");
+    return QRAF_HIP_OK;
+}
+static int copy_wait(void* dst, const void* src, size_t n, hipMemcpyKind kind) {
+    QH_TRY(not_capturing());
+    QH_CHECK_HIP(hipMemcpyWithStream(dst, src, n, kind, nullptr));
+    return QRAF_HIP_OK;
+}
+
+// Held by the engine while it captures a step, host work that waits for no other
+// thread, and by device synchronisation, which would break the capture.
+std::mutex& capture_mutex() {
+    static std::mutex* m = new std::mutex;  // outlives every thread
+    return *m;
+}
+
 // Staging buffer `i` of at least `bytes` on the current device (callers hold
 // g_mu, which serialises the buffers' use; g_dev_mu covers the lookup).
 static int staging(int i, size_t bytes, void** out) {
@@ -127,12 +149,10 @@ int qraf_hip_free(void* p) {
     return QRAF_HIP_OK;
 }
 int qraf_hip_memcpy_h2d(void* dst, const void* src, uint64_t n) {
-    if (n) QH_CHECK_HIP(hipMemcpy(dst, src, n, hipMemcpyHostToDevice));
-    return QRAF_HIP_OK;
+    return n ? copy_wait(dst, src, n, hipMemcpyHostToDevice) : QRAF_HIP_OK;
 }
 int qraf_hip_memcpy_d2h(void* dst, const void* src, uint64_t n) {
-    if (n) QH_CHECK_HIP(hipMemcpy(dst, src, n, hipMemcpyDeviceToHost));
-    return QRAF_HIP_OK;
+    return n ? copy_wait(dst, src, n, hipMemcpyDeviceToHost) : QRAF_HIP_OK;
 }
 int qraf_hip_memcpy_d2d(void* dst, const void* src, uint64_t n, void* stream) {
     if (n) QH_CHECK_HIP(hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToDevice, as_stream(stream)));
@@ -146,7 +166,9 @@ int qraf_hip_launch_floor_dev(int32_t workgroups, void* stream) {
     return qraf_hip::launch_empty(workgroups, as_stream(stream));
 }
 int qraf_hip_memset(void* p, int v, uint64_t n) {
-    if (n) QH_CHECK_HIP(hipMemset(p, v, n));
+    if (!n) return QRAF_HIP_OK;
+    QH_TRY(not_capturing());
+    QH_CHECK_HIP(hipMemsetAsync(p, v, n, nullptr));
     return QRAF_HIP_OK;
 }
 int qraf_hip_stream_create(void** s) {
@@ -165,6 +187,7 @@ int qraf_hip_stream_synchronize(void* s) {
     return QRAF_HIP_OK;
 }
 int qraf_hip_device_synchronize(void) {
+    std::lock_guard<std::mutex> lk(capture_mutex());
     QH_CHECK_HIP(hipDeviceSynchronize());
     return QRAF_HIP_OK;
 }
@@ -191,11 +214,13 @@ int qraf_hip_event_elapsed_ms(void* a, void* b, float* ms) {
 }
 int qraf_hip_graph_begin(void* s) {
     QH_CHECK_HIP(hipStreamBeginCapture(as_stream(s), hipStreamCaptureModeThreadLocal));
+    t_captures++;
     return QRAF_HIP_OK;
 }
 int qraf_hip_graph_end(void* s, void** exec) {
     QH_REQUIRE(exec, QRAF_HIP_ERR_INVALID, "null out pointer");
     hipGraph_t g;
+    if (t_captures > 0) t_captures--;
     QH_CHECK_HIP(hipStreamEndCapture(as_stream(s), &g));
     hipGraphExec_t ge;
     hipError_t e = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
@@ -228,10 +253,10 @@ int qraf_hip_register_weights(const void* host, uint64_t bytes) {
     }
     void* d = nullptr;
     QH_CHECK_HIP(hipMalloc(&d, bytes));
-    hipError_t e = hipMemcpy(d, host, bytes, hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
+    const int rc = copy_wait(d, host, bytes, hipMemcpyHostToDevice);
+    if (rc != QRAF_HIP_OK) {
         hipFree(d);
-        return set_error(QRAF_HIP_ERR_HIP, "weight upload failed: %s", hipGetErrorString(e));
+        return rc;
     }
     g_weights[host] = {d, bytes};
     return QRAF_HIP_OK;
@@ -257,8 +282,7 @@ static int device_weights(const void* host, size_t need, void** dev) {
         return QRAF_HIP_OK;
     }
     QH_TRY(staging(2, need, dev));
-    QH_CHECK_HIP(hipMemcpy(*dev, host, need, hipMemcpyHostToDevice));
-    return QRAF_HIP_OK;
+    return copy_wait(*dev, host, need, hipMemcpyHostToDevice);
 }
 
 int qraf_hip_matvec_q(const void* w, uint64_t w_size, uint32_t dtype, uint32_t block_size, uint32_t out_dim,

@@ -5,6 +5,7 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <mutex>
 #include <string>
 
 #include "../../include/qraf_hip.h"
@@ -242,6 +243,8 @@ __device__ __forceinline__ void wait_vm_lgkm0() {
 }
 
 
+// Held while the engine captures a step, and by the calls that would break it
+std::mutex& capture_mutex();
 // Library default stream of the current device (created by qraf_hip_init).
 hipStream_t default_stream();
 inline hipStream_t as_stream(void* s) { return s ? (hipStream_t)s : default_stream(); }

@@ -1367,9 +1367,11 @@ static int step_issue(qraf_engine* e, int32_t n, const int32_t* seq_ids, const u
         } else if (!g) {
             hipGraph_t graph = nullptr;
             e->stats.graph_captures += 1;
+            std::unique_lock<std::mutex> capturing(capture_mutex());
             QH_CHECK_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
             const int rc = enqueue(ctx_grid);
             const hipError_t ec = hipStreamEndCapture(s, &graph);
+            capturing.unlock();
             if (rc != QRAF_HIP_OK) {
                 if (graph) hipGraphDestroy(graph);
                 return rc;

@@ -785,6 +785,71 @@ def test_two_engines_in_two_threads(hip):
         m.close()
 
 
+def test_host_calls_while_another_thread_captures(hip):
+    """One thread captures step after step into graphs (every step count and
+    logit count twice, the second time captured) while another copies to and
+    from the device, clears memory, uploads weights and synchronises: no call
+    of either fails, every copy holds its bytes and every step its logits."""
+    import threading
+
+    from qraf_amd.backend import (DeviceBuffer, dispatch_matvec_q, register_weights, unregister_weights)
+    kw, seed = SMALL["q4_hd64_gqa2"]
+    m = oracle_model(kw, seed)
+    stop, errors, done = threading.Event(), [], {"copies": 0, "steps": 0}
+    wq = po.quantize(po.Q8_0, np.random.default_rng(1).standard_normal(64 * 256).astype(np.float32))
+    x = np.random.default_rng(2).standard_normal(256).astype(np.float32)
+    want_y = po.matvec_q(wq, po.Q8_0, 64, 256, x)
+
+    def host_calls():
+        try:
+            from qraf_amd.backend import backend_init
+            backend_init(0)
+            a = np.arange(100000, dtype=np.uint32)
+            buf = DeviceBuffer(a.nbytes)
+            y = np.zeros(64, np.float32)
+            while not stop.is_set():
+                buf.upload(a)
+                assert np.array_equal(buf.download(np.uint32, a.size), a)
+                buf.zero()
+                assert not buf.download(np.uint32, a.size).any()
+                dispatch_matvec_q(wq, wq.nbytes, po.Q8_0, None, 64, 256, x, y)  # uploads its weights
+                assert np.allclose(y, want_y, rtol=1e-4, atol=1e-4)
+                register_weights(wq)
+                unregister_weights(wq)
+                hip._lib.call("qraf_hip_device_synchronize")
+                done["copies"] += 1
+            buf.free()
+        except Exception as ex:  # noqa: BLE001
+            errors.append(repr(ex))
+
+    tf = upload(m, kw, max_batch=64)
+    e = tf.engine
+    t = threading.Thread(target=host_calls)
+    t.start()
+    try:
+        toks = [po.lib().or_gen_token(seed, i, kw["vocab"]) for i in range(48)]
+        e.set_row_padding(1)
+        for rnd in range(4):
+            for rows in range(1, 41, 3):
+                out = []
+                for _ in range(3):  # eager, captured, replayed
+                    sid = e.seq_create()
+                    lg, _ = e.step([sid] * rows, toks[:rows], list(range(rows)), logits=True)
+                    out.append(lg.copy())
+                    e.seq_release(sid)
+                    done["steps"] += 1
+                assert np.array_equal(out[0], out[1]) and np.array_equal(out[0], out[2])
+            e.set_fusion(6 if rnd % 2 else 7)  # drops the graphs: the next round captures again
+            e.set_graphs(False)
+            e.set_graphs(True)
+    finally:
+        stop.set()
+        t.join()
+        e.close()
+    assert not errors, errors[0]
+    assert done["copies"] > 0
+
+
 def test_1024_row_prefill_step(hip):
     """The engine's largest step: four 256-token prompts as one 1,024-row step
     (the gate/up GEMM with the SiLU-gate epilogue, every projection at 1,024
