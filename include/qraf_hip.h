@@ -54,7 +54,10 @@ int qraf_hip_device_count(int* count);
 /* Build information: "gfx950 <compiler version>". */
 const char* qraf_hip_version(void);
 
-/* Device memory, streams, events and graphs, so callers need no HIP headers. */
+/* Device memory, streams, events and graphs, so callers need no HIP headers.
+ * memcpy_h2d, memcpy_d2h and memset are complete on return and may be called
+ * while other threads capture graphs (a thread that captures is refused);
+ * device_synchronize only while no graph_begin of the caller's is open. */
 int qraf_hip_malloc(void** dev_ptr, uint64_t bytes);
 int qraf_hip_free(void* dev_ptr);
 int qraf_hip_memcpy_h2d(void* dst_dev, const void* src_host, uint64_t bytes);

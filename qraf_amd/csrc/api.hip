@@ -169,6 +169,8 @@ int qraf_hip_memset(void* p, int v, uint64_t n) {
     if (!n) return QRAF_HIP_OK;
     QH_TRY(not_capturing());
     QH_CHECK_HIP(hipMemsetAsync(p, v, n, nullptr));
+    // the library's streams do not wait for the legacy one
+    QH_CHECK_HIP(hipStreamSynchronize(nullptr));
     return QRAF_HIP_OK;
 }
 int qraf_hip_stream_create(void** s) {

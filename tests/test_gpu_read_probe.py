@@ -51,3 +51,20 @@ def test_launch_floor_runs_in_a_graph(hip, wgs):
     finally:
         g.destroy()
         s.destroy()
+
+
+def test_memset_is_complete_on_return(hip):
+    """A clear of 512 MB followed at once by a copy into its end on the
+    library's stream: the copy is there afterwards."""
+    from qraf_amd.backend import DeviceBuffer
+    n, m = 512 << 20, 4096
+    ones = np.arange(m, dtype=np.uint8) | 1
+    buf, src = DeviceBuffer(n), DeviceBuffer.from_array(ones)
+    for _ in range(4):
+        buf.zero()
+        hip._lib.call("qraf_hip_memcpy_d2d", buf.ptr + n - m, src.ptr, m, None)
+        hip._lib.call("qraf_hip_stream_synchronize", None)
+        assert np.array_equal(buf.download(np.uint8, m, n - m), ones)
+        assert not buf.download(np.uint8, m, 0).any()
+    buf.free()
+    src.free()
