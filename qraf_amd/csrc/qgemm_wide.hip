@@ -109,10 +109,9 @@ struct WideGeom {
     // W of stage it + WS, then X of stage it + NS - 1
     static constexpr int YOUNG = (NS - 2) * (XW + WI);
     static_assert(WS == NS - 1, "weights as far ahead as X");
-    static constexpr int PASS = NWV * TM * TN * 4096 > 128 * 1024 ? 2 : 1;  // SwiGLU epilogue's passes
-    static constexpr int RED = NWV * (TM / PASS) * TN * 4096;
+    static constexpr int RED = NWV * TM * TN * 4096;  // the SwiGLU epilogue: every wave's sums
     static constexpr int GIVE = WK == 2 ? TM * TN / 2 : TM * TN;  // tiles a wave hands to the other K groups
-    static_assert(TM % PASS == 0 && (WK == 1 || NWV * GIVE * 4096 <= RED), "epilogue");
+    static_assert(WK > 1 && NWV * GIVE * 4096 <= RED, "epilogue");
     static constexpr int LDS = LDS_X + LDS_W > RED ? LDS_X + LDS_W : RED;
     static_assert(LDS <= 160 * 1024, "LDS");
     static_assert(XI % WN == 0, "X split");
@@ -388,39 +387,35 @@ __global__ __launch_bounds__(64 * WN * WK, (WideGeom<FMT, TM, TN, WN, WK, NS, WS
         // tile q is finished by group q % WK and stored straight from registers:
         // bounds by the resource (rows) and the lane's offset (columns), so a store
         // is an add and the store itself
-        if constexpr (WK > 1) {
-            lds_barrier();
+        lds_barrier();
 #pragma unroll
-            for (int q = 0; q < U; q++)
-                if (q % WK != g)
+        for (int q = 0; q < U; q++)
+            if (q % WK != g)
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const float* a = acc[q / TN][q % TN] + 4 * i;
-                        red[((wave * G::GIVE + (WK == 2 ? q >> 1 : q)) * 4 + i) * 64 + lane] = f32x4{a[0], a[1], a[2], a[3]};
-                    }
-            __syncthreads();
-        }
+                for (int i = 0; i < 4; i++) {
+                    const float* a = acc[q / TN][q % TN] + 4 * i;
+                    red[((wave * G::GIVE + (WK == 2 ? q >> 1 : q)) * 4 + i) * 64 + lane] = f32x4{a[0], a[1], a[2], a[3]};
+                }
+        __syncthreads();
         const uint32_t rec = (uint32_t)(min(M - m0, G::MT) * N) * 4u;
         const rsrc_t yr = make_rsrc(Y + (size_t)split * slice + (size_t)m0 * N, rec);
         const rsrc_t ar = make_rsrc(add + (size_t)m0 * N, rec);
         const uint32_t rowb = (uint32_t)N * 4u;
 #pragma unroll
         for (int q = 0; q < U; q++) {
-            if (WK > 1 && q % WK != g) continue;
+            if (q % WK != g) continue;
             float(&a)[16] = acc[q / TN][q % TN];
-            if constexpr (WK > 1) {
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const f32x4 own = f32x4{a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3]};
-                    f32x4 v = own;
+            for (int i = 0; i < 4; i++) {
+                const f32x4 own = f32x4{a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3]};
+                f32x4 v = own;
 #pragma unroll
-                    for (int k = 0; k < WK; k++) {
-                        const f32x4 p = k == q % WK ? own : red[(((k * WN + wn) * G::GIVE + (WK == 2 ? q >> 1 : q)) * 4 + i) * 64 + lane];
-                        v = k ? v + p : p;
-                    }
-#pragma unroll
-                    for (int r = 0; r < 4; r++) a[4 * i + r] = v[r];
+                for (int k = 0; k < WK; k++) {
+                    const f32x4 p = k == q % WK ? own : red[(((k * WN + wn) * G::GIVE + (WK == 2 ? q >> 1 : q)) * 4 + i) * 64 + lane];
+                    v = k ? v + p : p;
                 }
+#pragma unroll
+                for (int r = 0; r < 4; r++) a[4 * i + r] = v[r];
             }
             const int n = n0 + 32 * (q % TN) + l32;
             const uint32_t at = n < N ? (uint32_t)n * 4u + (uint32_t)(4 * half) * rowb : 0x80000000u;
@@ -443,39 +438,34 @@ __global__ __launch_bounds__(64 * WN * WK, (WideGeom<FMT, TM, TN, WN, WK, NS, WS
     // SwiGLU: every wave's sums through LDS, then a loop over units of 4 rows of one
     // column (tile (t, u) of wave column w, rows 8 i + 4 half .. + 3)
     const int F2 = N >> 1;
-    constexpr int UP = U / G::PASS, UNITS = WN * UP * 4;  // tiles of a pass, units (of 64 lanes)
+    constexpr int UNITS = WN * U * 4;  // of 64 lanes
+    lds_barrier();                     // the stages are no longer read
 #pragma unroll
-    for (int pass = 0; pass < G::PASS; pass++) {
-        lds_barrier();  // the stages (the previous pass) are no longer read
+    for (int q = 0; q < U; q++)
 #pragma unroll
-        for (int q = 0; q < UP; q++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float* a = acc[(pass * UP + q) / TN][q % TN] + 4 * i;
-                red[((wave * UP + q) * 4 + i) * 64 + lane] = f32x4{a[0], a[1], a[2], a[3]};
-            }
-        __syncthreads();
+        for (int i = 0; i < 4; i++) {
+            const float* a = acc[q / TN][q % TN] + 4 * i;
+            red[((wave * U + q) * 4 + i) * 64 + lane] = f32x4{a[0], a[1], a[2], a[3]};
+        }
+    __syncthreads();
 #pragma unroll 2
-        for (int j = wave; j < UNITS; j += G::NWV) {
-            const int w = j / (UP * 4), q = (j >> 2) % UP, i = j & 3;
-            f32x4 v = red[j * 64 + lane];
+    for (int j = wave; j < UNITS; j += G::NWV) {
+        const int w = j / (U * 4), q = (j >> 2) % U, i = j & 3;
+        f32x4 v = red[j * 64 + lane];
 #pragma unroll
-            for (int k = 1; k < WK; k++) v += red[(k * UNITS + j) * 64 + lane];
-            const int n = tile * G::NT + w * 32 * TN + 32 * (q % TN) + l32;
-            const int m = m0 + 32 * ((pass * UP + q) / TN) + 8 * i + 4 * half;
-            {
-                // gate and up columns in neighbouring lanes: the even lane takes rows 0 and 2, the odd lane 1 and 3
-                const bool odd = lane & 1;
+        for (int k = 1; k < WK; k++) v += red[(k * UNITS + j) * 64 + lane];
+        const int n = tile * G::NT + w * 32 * TN + 32 * (q % TN) + l32;
+        const int m = m0 + 32 * (q / TN) + 8 * i + 4 * half;
+        // gate and up columns in neighbouring lanes: the even lane takes rows 0 and 2, the odd lane 1 and 3
+        const bool odd = lane & 1;
 #pragma unroll
-                for (int r = 0; r < 4; r += 2) {
-                    const float give = odd ? v[r] : v[r + 1], got = __shfl_xor(give, 1);
-                    const float gate = odd ? got : v[r], up = odd ? v[r + 1] : got;
-                    const int mm = m + r + (odd ? 1 : 0);
-                    if (mm < M && n < N) {
-                        const size_t e = (size_t)mm * F2 + (n >> 1);
-                        split_bf16(silu_gate(gate, up), &act_hi[e], &act_lo[e]);
-                    }
-                }
+        for (int r = 0; r < 4; r += 2) {
+            const float give = odd ? v[r] : v[r + 1], got = __shfl_xor(give, 1);
+            const float gate = odd ? got : v[r], up = odd ? v[r + 1] : got;
+            const int mm = m + r + (odd ? 1 : 0);
+            if (mm < M && n < N) {
+                const size_t e = (size_t)mm * F2 + (n >> 1);
+                split_bf16(silu_gate(gate, up), &act_hi[e], &act_lo[e]);
             }
         }
     }
