@@ -275,8 +275,9 @@ int qraf_hip_set_qgemm_schedule(int32_t mode, int32_t min_blocks);
 /* Wave-split form of the tile-major GEMM (each workgroup's 4 waves take its
  * quant blocks in turn and meet once in LDS at the end): mode 1 selects it
  * for every tiled batch over 16 rows, -1 never, 0 (the default) for batches
- * of 17-32 rows where the 32x32 form (the automatic choice of most batches
- * over 16 rows while no form or split count is forced) does not run, unless
+ * of 17-64 rows (over 32 of less than 16384 weight rows) where the 32x32 form
+ * (the automatic choice of most batches over 16 rows while no form or split
+ * count is forced) does not run, unless
  * qraf_hip_set_qgemm_tuning forces another form;
  * tiles_per_workgroup 2, 3 or 4 fixes its 16-row weight tiles per workgroup
  * (0: automatic).  Affects the workspace queries and the SwiGLU-epilogue
@@ -338,9 +339,9 @@ int qraf_hip_qgemm_tiled_argmax_dev(const void* w_tiled, uint32_t dtype, uint32_
  * 2i = gate_i, row 2i+1 = up_i, out_dim = 2F, even); out_hi/out_lo [batch][F]
  * receive silu(gate) * up as the hi/lo planes the down projection's GEMM
  * reads (qraf_hip_split_bf16_dev form; they must not overlap x_hi/x_lo).
- * The pipelined kernel runs unsplit (128 weight rows x 64 batch rows per
- * workgroup), so no workspace is needed and the gate/up sums never leave the
- * registers; the sums are those of qraf_hip_qgemm_tiled_dev in the same form.
+ * The kernel runs unsplit, so no workspace is needed and the gate/up sums
+ * never leave the registers; they are those of qraf_hip_qgemm_tiled_dev in
+ * the same form and one split.
  * No counterpart in the reference (a fusion of two of its steps). */
 int qraf_hip_qgemm_tiled_silu_dev(const void* w_tiled, uint32_t dtype, uint32_t out_dim, uint32_t in_dim,
                                   const uint16_t* x_hi, const uint16_t* x_lo, int32_t batch, uint16_t* out_hi,

@@ -1417,15 +1417,14 @@ static void qgemm_stream(QgPlan& p, int nb, int slots) {
     p.S = smax;
 }
 
-// The wave-split kernel for a tiled N x K product of M rows.  Automatic
-// choice (MI355X, Q4_0 and Q8_0 at the Qwen2.5-3B shapes, GEMM + partial sums,
-// graph-timed): batches of 17-32 rows on every shape (Q4 11008 x 2048 14.8 us
-// against 20.8 for the 32-row-chunk kernel, 2048 x 2048 8.3 against 12.2) and
-// of 33-64 rows below 16384 weight rows (11008 x 2048 23.0 against 25.7, 2048 x
-// 11008 22.7 against 28.9); from 65 rows, and for the 22016-row gate/up
-// product at 33-64 rows (42.1 against 37.4), the LDS-shared pipelined kernels,
-// whose X fragments each feed 8 waves (here each wave reads its own: 5x the X
-// bytes per MFMA at 128 rows, 40-83 us against 29-49).
+// The wave-split kernel for a tiled N x K product of M rows that the 32x32 kernel
+// does not take (wide_wanted): batches of 17-32 rows on every shape (Q4 11008 x
+// 2048 14.8 us against 20.8 for the 32-row-chunk kernel, 2048 x 2048 8.3 against
+// 12.2) and of 33-64 rows below 16384 weight rows (11008 x 2048 23.0 against 25.7,
+// 2048 x 11008 22.7 against 28.9).  Otherwise the LDS-shared kernels, whose X
+// fragments each feed several waves (here each wave reads its own: 5x the X
+// bytes per MFMA at 128 rows, 40-83 us against 29-49; the 22016-row gate/up
+// product at 33-64 rows 42.1 against 37.4).
 static bool kw_wanted(int N, int M) {
     if (g_qg_kw < 0 || (g_qg_pipe != 0 && g_qg_kw == 0)) return false;  // an older form forced
     if (g_qg_kw > 0) return M > 16;
@@ -1498,14 +1497,14 @@ static void kx_plan(QgPlan& p, int N, int nb, int M, bool whole) {
     p.ws_bytes = p.S > 1 ? (size_t)p.S * M * N * 4 : 0;
 }
 
-// The row-split LDS-shared kernel where it measured faster than the other
-// forms (MI355X, tiled, GEMM + partial sums, graph-timed): 33-64 rows on
-// products of 16384 rows and more (Q4 22016 x 2048 at 64 rows 29.9 us against
-// 38.3 for the pipelined kernel and 42.1 for the wave-split one), and Q8_0
-// products with a long in_dim from 65 rows (2048 x 11008 at 128 / 256 rows
-// 34.1 / 54.9 against 41.8 / 65.2); the SwiGLU-epilogue entry from 256 rows
-// (22016 x 2048 at 256 rows: Q4 78.7 against 84.7, Q8 81.1 against 122.7).
-// At 128 rows on the Q4 shapes it ties or trails the pipelined kernel.
+// The row-split LDS-shared kernel, of the products that the 32x32 kernel does not
+// take, where it measured faster than the other forms (MI355X, tiled, GEMM +
+// partial sums, graph-timed): 33-64 rows on products of 16384 rows and more (Q4
+// 22016 x 2048 at 64 rows 29.9 us against 38.3 for the pipelined kernel and 42.1 for
+// the wave-split one), and Q8_0 products with a long in_dim from 65 rows (2048 x
+// 11008 at 128 / 256 rows 34.1 / 54.9 against 41.8 / 65.2); the SwiGLU-epilogue entry
+// from 256 rows (22016 x 2048 at 256 rows: Q4 78.7 against 84.7, Q8 81.1 against
+// 122.7).  At 128 rows on the Q4 shapes it ties or trails the pipelined kernel.
 static bool kx_wanted(uint32_t dtype, int N, int K, int M) {
     if (g_qg_pipe == 3) return M > 16;
     if (g_qg_pipe != 0 || g_qg_kw != 0) return false;
@@ -1525,7 +1524,7 @@ static double qg_rounds(long long W, int slots, double part) {
 // is returned.  Rounds of workgroups (one per CU; the Q4_0 64 x 128 tile leaves
 // room for two, which then share the CU) x (us an iteration of WK pairs of
 // blocks x iterations + us to start and finish, longer for the SwiGLU epilogue)
-// + the launch + the traffic of the partial slices.  Fitted to 43,000 timings of
+// + the launch + the traffic of the partial slices.  Fitted to 56,000 timings of
 // every form and split on MI355X (17-1,024 rows, N 576-151936, K 256-18944):
 // median error 2-5%; the plan it picks is 0.3% off the best of them on average.
 static double wide_plan(QgPlan& p, uint32_t dtype, int N, int nb, int M, bool whole) {
@@ -2160,10 +2159,11 @@ int launch_qgemm_argmax(const void* Wt, uint32_t dtype, int N, int K, const uint
     return QRAF_HIP_OK;
 }
 
-// Gate/up projection of interleaved rows with the SwiGLU front in the
-// epilogue: the narrow pipelined form (4 waves x 128 weight rows, 64-row
-// batch chunks, one workgroup per (tile, chunk), no split) so that every
-// workgroup holds complete sums; act_hi/act_lo [M][N/2] must not overlap xh/xl.
+// Gate/up projection of interleaved rows with the SwiGLU front in the epilogue,
+// unsplit so that every workgroup holds complete sums: the 32x32 kernel where
+// wide_wanted, else the row-split kernel from 256 rows, the wave-split one up to
+// 64, and the narrow pipelined form (4 waves x 128 weight rows, 64-row batch
+// chunks); act_hi/act_lo [M][N/2] must not overlap xh/xl.
 int launch_qgemm_silu(const void* Wt, uint32_t dtype, int N, int K, const uint16_t* xh, const uint16_t* xl, int M,
                       uint16_t* act_hi, uint16_t* act_lo, hipStream_t s) {
     QH_REQUIRE(dtype == DT_Q8_0 || dtype == DT_Q4_0, QRAF_HIP_ERR_DTYPE, "qgemm silu: unsupported dtype %u", dtype);

@@ -15,16 +15,18 @@
 // WS of the wave's own weights; one barrier per pair (none for WN = 1).
 //
 // 32x32x16 products and not 16x16x32: an X fragment read from LDS serves twice the
-// outputs, and one wave per SIMD keeps the matrix cores busy (2,247 TFLOP/s
-// against 1,183 with 8 independent 16x16 accumulators, registers only).  What
-// bounds the loop is the vector ALU beside them: per unit of four products (a 32 x
-// 32 tile of one block, 128 matrix cycles) 16 scale FMAs, 18 (TM 2) or 9 (TM 4) of
-// the weights' conversion; measured 1.15 us an iteration of TM 2 (8 units) and 1.6
-// of TM 4 (16 units) at one wave per SIMD, 45-54% of the matrix rate.  Against the
-// forms of qgemm.hip (MI355X, GEMM and partial sums, Q4_0): 11008 x 2048 at 32 /
-// 64 / 128 rows 14.2 / 21.9 / 30.1 -> 10.8 / 14.4 / 23.2 us, 2560 x 2048 at 128 rows
-// 16.0 -> 10.3, 2048 x 11008 at 128 / 512 rows 26.7 / 63.2 -> 23.7 / 54.2; Q8_0 2048 x
-// 11008 at 203 rows 52.1 -> 33.6.
+// outputs (registers only, 8 independent accumulators: 2,247 TFLOP/s against 1,183).
+// What bounds the loop is the vector ALU beside them: per unit of four products (a
+// 32 x 32 tile of one block, 128 matrix cycles) 16 scale FMAs, 18 (TM 2) or 9 (TM 4)
+// of the weights' conversion, which overlap the products only in part.  An iteration
+// of 4 / 8 / 16 units takes 0.8-0.9 / 1.1-1.4 / 1.6-1.75 us at TM 1 / 2 / 4, that is 25 /
+// 31-39 / 49-53% of the matrix rate; over the whole launch (MI355X, Q4_0 11008 x 2048 at
+// 128 rows, 24.2 us) the products take 30% of the waves' cycles, the VALU issues in
+// 42% (in two fifths of the products' cycles) and 31% wait for LDS, memory or the
+// barrier.  Against the forms of qgemm.hip (MI355X, GEMM and partial sums, Q4_0):
+// 11008 x 2048 at 32 / 64 / 128 rows 14.2 / 21.9 / 30.1 -> 10.8 / 14.4 / 23.2 us, 2560 x 2048
+// at 128 rows 16.0 -> 10.3, 2048 x 11008 at 128 / 512 rows 26.7 / 63.2 -> 23.7 / 54.2; Q8_0
+// 2048 x 11008 at 203 rows 52.1 -> 33.6.
 #include <type_traits>
 
 #include "common.h"
