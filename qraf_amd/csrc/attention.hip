@@ -1004,12 +1004,13 @@ __global__ __launch_bounds__(64 * NW, NW == 12 ? 3 : 4) void attn_mfma_kernel(At
         }
     } else {
 #pragma unroll
-    for (int d = 0; d < DT; d++)
+    for (int r = 0; r < 4; r++) {  // the row outside: one predicate and one address for a row's stores
+        const int h = 4 * seg + r;
+        float* row = &s_o[wave * G + h][l16];
+        if (h < G && (NW == 4 || active))
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int h = 4 * seg + r;
-            if (h < G && (NW == 4 || active)) s_o[wave * G + h][16 * d + l16] = o[d][r] * ounit;
-        }
+            for (int d = 0; d < DT; d++) row[16 * d] = o[d][r] * ounit;
+    }
     }
     __syncthreads();
     const int na = NW == 4 ? 4 : min(NW, (ctx - chunk * CH + 63) >> 6);  // waves with positions
