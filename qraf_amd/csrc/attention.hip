@@ -328,8 +328,12 @@ __global__ __launch_bounds__(ACH) void attn_decode_kernel(AttnArgs a) {
 // 16.  Every exchange is DPP or a lane-row swap: with 16 waves on one CU the
 // LDS shuffles took longer than the loads (4 heads, 256 positions, one sequence: 7.9 us with
 // LDS shuffles, 6.7 with these, 4.2 with a workgroup per head).
-// Positions past the context read the tile's first row and count as 0, as do
-// scores of -inf: a wave may hold nothing else.
+// Positions past the context read the tile's first row for K and zeros for V (a
+// row of the cache could hold an infinity, and 0 times it is NaN) and count as
+// 0, as do scores of -inf: a wave may hold nothing else.  Pointing the lane at
+// zeros costs no instruction over pointing it at a row; zeroing what it loaded
+// took 3.42 us instead of 3.24 (9/3 heads of 64, 161 positions, warm) and
+// 4.23 instead of 3.88 inside a step, where the code is not in the caches.
 // ---------------------------------------------------------------------------
 // lane exchanges without LDS: DPP controls inside rows of 16 lanes (quad_perm
 // for xor 1 and 2, row_ror, row_newbcast), lane-row swaps across them
@@ -354,6 +358,12 @@ __device__ __forceinline__ float over_rows(float x, float y, float z, float w, F
     const auto c = __builtin_amdgcn_permlane32_swap(u(p), u(q), false, false);
     return op(f(c[0]), f(c[1]));
 }
+__device__ const float g_zero_row[128] = {};
+// named global: loads through a pointer chosen from two objects would be flat ones
+typedef float f4_raw __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(1))) f4_raw GlobalF4;
+// a maximum to subtract: scores that are all -inf stay -inf, and count as 0
+__device__ __forceinline__ float finite_max(float m) { return m == -INFINITY ? 0.f : m; }
 template <int HD, int G, int TPW>
 __global__ __launch_bounds__(1024, 4) void attn_few_kernel(AttnArgs a) {
     constexpr int NW = 16, KQ = HD / 16, VQ = HD / 64;  // float4s of a lane's K quarter, of its V dimensions
@@ -388,19 +398,18 @@ __global__ __launch_bounds__(1024, 4) void attn_few_kernel(AttnArgs a) {
     for (int t = 0; t < TPW; t++) {
         const int p0 = 16 * (wave + NW * t);
         if (p0 < ctx) {  // wave-uniform
-            // row of position p0 + x on page id; past the context p0's row
+            // row of position p on page id; past the context K reads p0's row, V zeros
             const int first = __builtin_amdgcn_readfirstlane(pg[t]);
-            auto row = [&](int x, int id) {
-                const bool in = p0 + x < ctx;
-                return (((size_t)(in ? id : first) * a.Hkv + kvh) * a.page_size + (in ? p0 + x : p0) % a.page_size) * HD;
-            };
-            const float* kp = kc + row(i, pg[t]) + 4 * j;
+            auto row = [&](int p, int id) { return (((size_t)id * a.Hkv + kvh) * a.page_size + p % a.page_size) * HD; };
+            const bool in = p0 + i < ctx;
+            const float* kp = kc + row(in ? p0 + i : p0, in ? pg[t] : first) + 4 * j;
 #pragma unroll
             for (int k = 0; k < KQ; k++) kr[t][k] = *(const float4*)(kp + 16 * k);
             auto vrow = [&](int x, int id, float4 (&v)[VQ]) {
-                const float* vp = vc + row(x, id) + 4 * c;
+                const uint64_t at = (uint64_t)(vc + row(p0 + x, id));
+                const uint64_t vp = (p0 + x < ctx ? at : (uint64_t)g_zero_row) + 16 * c;
 #pragma unroll
-                for (int y = 0; y < VQ; y++) v[y] = *(const float4*)(vp + 64 * y);
+                for (int y = 0; y < VQ; y++) v[y] = __builtin_bit_cast(float4, *((const GlobalF4*)vp + 16 * y));
             };
             vrow(4 * r + 0, dpp<DPP_BCAST + 0>(pg[t]), vr[t][0]);
             vrow(4 * r + 1, dpp<DPP_BCAST + 4>(pg[t]), vr[t][1]);
@@ -445,20 +454,14 @@ __global__ __launch_bounds__(1024, 4) void attn_few_kernel(AttnArgs a) {
     mx = fmaxf(mx, dpp<DPP_ROR8>(mx));  // row h: head h's maximum
 #pragma unroll
     for (int h = 0; h < G; h++)
-        m[h] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mx), 16 * h));
+        m[h] = finite_max(__builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mx), 16 * h)));
 #pragma unroll
     for (int t = 0; t < TPW; t++) {
         const int p0 = 16 * (wave + NW * t);
         if (p0 < ctx) {
-            if (p0 + 16 > ctx)  // the first row's repetitions: 0 times an infinity would be NaN
-#pragma unroll
-                for (int x = 0; x < 4; x++)
-#pragma unroll
-                    for (int y = 0; y < VQ; y++)
-                        if (p0 + 4 * r + x >= ctx) vr[t][x][y] = float4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int h = 0; h < G; h++) {
-                const float p = sc[t][h] == -INFINITY ? 0.f : __expf(sc[t][h] - m[h]);  // m may be -inf
+                const float p = __expf(sc[t][h] - m[h]);
                 l[h] += p;
                 auto add = [&](float w, const float4 (&v)[VQ]) {
 #pragma unroll
@@ -497,9 +500,10 @@ __global__ __launch_bounds__(1024, 4) void attn_few_kernel(AttnArgs a) {
     const int nw = min(NW, (ctx + 15) >> 4);  // waves with positions
     float M = s_m[0][h];
     for (int v = 1; v < nw; v++) M = fmaxf(M, s_m[v][h]);
+    M = finite_max(M);
     float O = 0.f, L = 0.f;
     for (int v = 0; v < nw; v++) {
-        const float e = s_m[v][h] == -INFINITY ? 0.f : __expf(s_m[v][h] - M);
+        const float e = __expf(s_m[v][h] - M);
         O = __builtin_fmaf(s_o[v][h][d], e, O);
         L = __builtin_fmaf(s_l[v][h], e, L);
     }
